@@ -35,10 +35,10 @@ __device__ __forceinline__ uint32_t perm_b32(uint32_t hi_src, uint32_t lo_src, u
 }
 
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  const __bf16 a = (__bf16)lo;  // round to nearest even
-  const __bf16 b = (__bf16)hi;
-  return (uint32_t)__builtin_bit_cast(uint16_t, a) |
-         ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+  // Round to nearest even, as one v_cvt_pk_bf16_f32.
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 
 __device__ __forceinline__ float bf16_lo(uint32_t pair) {
