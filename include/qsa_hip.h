@@ -462,6 +462,18 @@ int qsa_gdn_recurrence(const float* q, const float* k, const void* v, const floa
                        int key_heads, int value_heads, int head_dim, int max_seq_tokens, void* o,
                        void* stream);
 
+/* The same with a workspace for the two-launch chunked kernels, which spread a
+ * long sequence over many compute units. Bytes needed (0: the call uses none,
+ * as for a decode batch). A null workspace, or an o that is not 16-byte aligned,
+ * runs qsa_gdn_recurrence's kernels. */
+size_t qsa_gdn_recurrence_workspace_bytes(int tokens, int num_seqs, int key_heads, int value_heads,
+                                          int max_seq_tokens);
+int qsa_gdn_recurrence_ws(const float* q, const float* k, const void* v, const float* g,
+                       const float* beta, int tokens, float* state, int num_slots,
+                       const int32_t* query_start_loc, const int64_t* slots, int num_seqs,
+                       int key_heads, int value_heads, int head_dim, int max_seq_tokens, void* o,
+                       void* workspace, size_t workspace_bytes, void* stream);
+
 /* Gated RMSNorm of the GDN output: y = bf16(rmsnorm(o) * weight * silu(z)) per
  * (token, value head), z read from the qkvz projection rows. Tensors 16-byte
  * aligned, qkvz_stride a multiple of 8 elements. */

@@ -171,6 +171,10 @@ SIGNATURES = {
     "qsa_gdn_recurrence": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i32, c_ptr, c_i32,
                                    c_ptr, c_ptr, c_i32, c_i32, c_i32, c_i32, c_i32, c_ptr,
                                    c_ptr]),
+    "qsa_gdn_recurrence_workspace_bytes": (c_size, [c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "qsa_gdn_recurrence_ws": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i32, c_ptr, c_i32,
+                                      c_ptr, c_ptr, c_i32, c_i32, c_i32, c_i32, c_i32, c_ptr,
+                                      c_ptr, c_size, c_ptr]),
     "qsa_gdn_gated_norm": (c_i32, [c_ptr, c_ptr, c_i64, c_ptr, ctypes.c_float, c_i32, c_i32,
                                    c_i32, c_i32, c_ptr, c_ptr]),
 }

@@ -30,7 +30,7 @@
 // per key head); the conv channels are ordered [q of all key heads, k of all
 // key heads, v of all value heads]; conv state [slots, K-1, channels] bf16
 // (oldest row first); recurrent state [slots, value heads, 128, 128] fp32.
-#include "qsa_common.h"
+#include "gdn_args.h"
 #include "../../include/qsa_hip.h"
 
 namespace qsa {
@@ -539,21 +539,6 @@ __global__ __launch_bounds__(256) void gdn_conv_state_kernel(const GdnConvStateA
 }
 
 constexpr int kRecTokens = 16;  // tokens staged in LDS per block
-constexpr int kChunkMin = 16;   // sequences this long take gdn_chunk_kernel
-
-struct GdnRecurArgs {
-  const float* q;  // [tokens, key_heads, 128]
-  const float* k;
-  const uint16_t* v;  // [tokens, value_heads, 128]
-  const float* g;     // [tokens, value_heads]
-  const float* beta;
-  float* state;  // [slots, value_heads, 128, 128]
-  const int* seq_start;
-  const int64_t* slots;
-  int num_seqs, key_heads, value_heads, num_slots, tokens;
-  uint16_t* o;  // [tokens, value_heads, 128]
-  int chunk_min;  // sequences this long go to gdn_chunk_kernel, shorter ones to the per-token kernel
-};
 
 __global__ __launch_bounds__(256) void gdn_recurrence_kernel(const GdnRecurArgs a) {
   __shared__ float sq[kRecTokens][kHeadDim];
@@ -647,7 +632,7 @@ __global__ __launch_bounds__(256) void gdn_recurrence_kernel(const GdnRecurArgs 
 }
 
 // ---------------------------------------------------------------------------
-// Chunked gated delta rule (sequences of kChunkMin tokens or more).
+// Chunked gated delta rule (sequences of kGdnChunkMin tokens or more).
 //
 // The recurrence over a chunk of C = 64 tokens in its WY form. With G the
 // in-chunk cumulative log decay, gamma = e^G and S the state at the chunk
@@ -1180,11 +1165,15 @@ extern "C" int qsa_gdn_conv_state(const void* qkvz, int64_t qkvz_stride, int tok
   return check_launch("qsa_gdn_conv_state");
 }
 
-extern "C" int qsa_gdn_recurrence(const float* q, const float* k, const void* v, const float* g,
-                                  const float* beta, int tokens, float* state, int num_slots,
-                                  const int* query_start_loc, const int64_t* slots, int num_seqs,
-                                  int key_heads, int value_heads, int head_dim,
-                                  int max_seq_tokens, void* o, void* stream) {
+namespace {
+// The two-launch form's workspace past this bound is not asked for: the
+// one-launch kernel needs none.
+constexpr size_t kScanWorkspaceMax = (size_t)2 << 30;
+
+int gdn_recurrence(const float* q, const float* k, const void* v, const float* g, const float* beta,
+                   int tokens, float* state, int num_slots, const int* query_start_loc,
+                   const int64_t* slots, int num_seqs, int key_heads, int value_heads, int head_dim,
+                   int max_seq_tokens, void* o, void* workspace, size_t workspace_bytes, void* stream) {
   GdnShape s;
   if (!gdn_shape(key_heads, value_heads, head_dim, 4, &s, "qsa_gdn_recurrence")) return QSA_ERR_UNSUPPORTED;
   if (num_seqs < 0 || tokens < 0) return fail(QSA_ERR_INVALID, "qsa_gdn_recurrence: negative size");
@@ -1195,23 +1184,64 @@ extern "C" int qsa_gdn_recurrence(const float* q, const float* k, const void* v,
     return fail(QSA_ERR_INVALID, "qsa_gdn_recurrence: tensors must be 16-byte aligned");
   if ((int64_t)num_seqs * value_heads > 0x7fffffffLL)
     return fail(QSA_ERR_UNSUPPORTED, "qsa_gdn_recurrence: too many (sequence, head) pairs");
-  // With no sequence of kChunkMin tokens (a decode batch, as the caller
-  // states), the chunked kernel is not launched and the per-token kernel
-  // takes every sequence, whatever its length: a wrong bound costs time only.
-  const bool chunks = max_seq_tokens < 0 || max_seq_tokens >= kChunkMin;
+  // With no sequence of kGdnChunkMin tokens (a decode batch, as the caller
+  // states), no chunked kernel is launched and the per-token kernel takes
+  // every sequence, whatever its length: a wrong bound costs time only.
+  const bool chunks = max_seq_tokens < 0 || max_seq_tokens >= kGdnChunkMin;
   GdnRecurArgs a{q, k, static_cast<const uint16_t*>(v), g, beta, state, query_start_loc, slots,
                  num_seqs, key_heads, value_heads, num_slots, tokens, static_cast<uint16_t*>(o),
-                 chunks ? kChunkMin : 0x7fffffff};
+                 chunks ? kGdnChunkMin : 0x7fffffff};
+  hipStream_t st = static_cast<hipStream_t>(stream);
   if (chunks) {
     // Long sequences (chunks) first on the stream: their workgroups are the long ones.
-    hipLaunchKernelGGL(gdn_chunk_kernel, dim3(num_seqs * value_heads), dim3(256), sizeof(ChunkLds),
-                       static_cast<hipStream_t>(stream), a);
-    const int st = check_launch("qsa_gdn_recurrence (chunks)");
-    if (st != QSA_OK) return st;
+    const size_t need = qsa_gdn_recurrence_workspace_bytes(tokens, num_seqs, key_heads, value_heads, max_seq_tokens);
+    int rc;
+    if (workspace && need && aligned16(o)) {
+      if (workspace_bytes < need || !aligned16(workspace))
+        return fail(QSA_ERR_WORKSPACE, "qsa_gdn_recurrence: workspace too small or not 16-byte aligned");
+      rc = gdn_scan_launch(a, max_seq_tokens, workspace, st);
+    } else {
+      hipLaunchKernelGGL(gdn_chunk_kernel, dim3(num_seqs * value_heads), dim3(256), sizeof(ChunkLds), st, a);
+      rc = check_launch("qsa_gdn_recurrence (chunks)");
+    }
+    if (rc != QSA_OK) return rc;
   }
-  hipLaunchKernelGGL(gdn_recurrence_kernel, dim3(num_seqs * value_heads), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(gdn_recurrence_kernel, dim3(num_seqs * value_heads), dim3(256), 0, st, a);
   return check_launch("qsa_gdn_recurrence");
+}
+}  // namespace
+
+extern "C" size_t qsa_gdn_recurrence_workspace_bytes(int tokens, int num_seqs, int key_heads,
+                                                     int value_heads, int max_seq_tokens) {
+  // Sequences of a single chunk stay on the one-launch kernel: there is nothing
+  // to walk, and it saves the operands' round trip through memory (16 of 60
+  // tokens 25 us against 40, 64 of 60 tokens 91 against 94).
+  if (tokens <= 0 || num_seqs <= 0 || key_heads <= 0 || value_heads <= 0 || tokens <= kChunk ||
+      (max_seq_tokens >= 0 && max_seq_tokens <= kChunk) ||
+      (int64_t)num_seqs * value_heads > 0x7fffffffLL / 8 || (int64_t)num_seqs + tokens > 0x7fffffffLL)
+    return 0;
+  const size_t bytes = gdn_scan_workspace_bytes(tokens, num_seqs, key_heads, value_heads);
+  return bytes <= kScanWorkspaceMax ? bytes : 0;
+}
+
+extern "C" int qsa_gdn_recurrence(const float* q, const float* k, const void* v, const float* g,
+                                  const float* beta, int tokens, float* state, int num_slots,
+                                  const int* query_start_loc, const int64_t* slots, int num_seqs,
+                                  int key_heads, int value_heads, int head_dim,
+                                  int max_seq_tokens, void* o, void* stream) {
+  return gdn_recurrence(q, k, v, g, beta, tokens, state, num_slots, query_start_loc, slots, num_seqs,
+                        key_heads, value_heads, head_dim, max_seq_tokens, o, nullptr, 0, stream);
+}
+
+extern "C" int qsa_gdn_recurrence_ws(const float* q, const float* k, const void* v, const float* g,
+                                     const float* beta, int tokens, float* state, int num_slots,
+                                     const int* query_start_loc, const int64_t* slots, int num_seqs,
+                                     int key_heads, int value_heads, int head_dim,
+                                     int max_seq_tokens, void* o, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  return gdn_recurrence(q, k, v, g, beta, tokens, state, num_slots, query_start_loc, slots, num_seqs,
+                        key_heads, value_heads, head_dim, max_seq_tokens, o, workspace, workspace_bytes,
+                        stream);
 }
 
 extern "C" int qsa_gdn_gated_norm(const void* o, const void* qkvz, int64_t qkvz_stride,

@@ -526,3 +526,49 @@ def test_recorded_gemm_choices_load_and_agree_with_library_default():
         scale = b.float().abs().max().item()
         print(f"[hybrid] recorded GEMM {m}x{n}x{k}: max diff {err:.3e} of {scale:.3e}", flush=True)
         assert err <= 0.02 * scale
+
+
+@pytest.mark.parametrize("hk,hv,lens,bound", [
+    (2, 2, [16, 63, 15, 64, 65, 300], None),        # narrow slices, three buffers; r = 1
+    (2, 6, [129, 1, 192, 17, 16, 70, 40, 64], None),  # two narrow slices a workgroup; r = 3
+    (8, 16, [200, 128, 16, 1, 90, 66], None),       # wide slices
+    (8, 16, [700], 700),                            # one sequence, narrow slices
+    (2, 4, [64, 16, 33, 2], 64),                    # single chunks: the one-launch kernel
+])
+def test_gdn_recurrence_chunk_edges(hk, hv, lens, bound):
+    """Every launch of the chunked delta rule at its edges: sequences of a chunk
+    less one, one and one more token, padding slots between sequences, a
+    sequence without a state slot, and one whose range leaves the batch (skipped:
+    its state and the rows past the batch stay as they are). Error bound of the
+    bf16 products over a chunk: as the length-bound test above."""
+    gen = torch.Generator().manual_seed(sum(lens) + hv)
+    tokens = sum(lens)
+    q = torch.nn.functional.normalize(torch.randn(tokens, hk, 128, generator=gen), dim=-1) / 128 ** 0.5
+    k = torch.nn.functional.normalize(torch.randn(tokens, hk, 128, generator=gen), dim=-1)
+    v = torch.randn(tokens, hv, 128, generator=gen).to(torch.bfloat16)
+    g = -0.5 * torch.rand(tokens, hv, generator=gen)
+    beta = torch.rand(tokens, hv, generator=gen)
+    n = len(lens)
+    state0 = 0.05 * torch.randn(n + 2, hv, 128, 128, generator=gen)
+    starts = torch.tensor([0] + np.cumsum(lens).tolist() + [tokens + 100], dtype=torch.int32)
+    slots = torch.randperm(n + 2, generator=gen)[:n + 1]
+    without = int(np.argmax(lens))
+    slots[without] = -1
+    state = state0.to(DEV)
+    print(f"[hybrid] gdn recurrence, {hk}/{hv} heads, {lens}, bound {bound}", flush=True)
+    o = L.gdn_recurrence(q.to(DEV), k.to(DEV), v.to(DEV), g.to(DEV), beta.to(DEV), state,
+                         starts.to(DEV), slots.to(DEV), hk, hv, max_query_len=bound)
+    torch.cuda.synchronize()
+    kh = torch.arange(hv) // (hv // hk)
+    untouched = set(range(n + 2))
+    for i, m in enumerate(lens):
+        rows, slot = slice(int(starts[i]), int(starts[i]) + m), int(slots[i])
+        s0 = torch.zeros(hv, 128, 128) if i == without else state0[slot]
+        want_o, want_s = H.gated_delta_rule(q[rows][:, kh], k[rows][:, kh], v[rows].float(),
+                                            g[rows], beta[rows], s0)
+        _close(o[rows].cpu(), want_o, f"output, sequence of {m}")
+        if i != without:
+            untouched.remove(slot)
+            _close(state[slot].cpu(), want_s, f"state, sequence of {m}", 1e-2, 1e-3)
+    for slot in untouched:
+        assert torch.equal(state[slot].cpu(), state0[slot])
