@@ -64,6 +64,15 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
   return v;
 }
 
+// c + a[0] b[0] + a[1] b[1] of bf16 pairs, in fp32.
+__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
+}
+
+// Every element rounded to bf16, two at a time (one conversion for a pair).
+__device__ __forceinline__ void round8(float (&f)[8]) { unpack8(pack8(f), f); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
@@ -86,8 +95,23 @@ __device__ __forceinline__ float wave_sum(float v) {
 //    so the accumulator lands in the lane that holds n for the same
 //    (token, column) and the epilogue needs no exchange. The rank-16 K
 //    dimension is padded to 32 with zero lanes (g >= 2).
-// Weights are read once per 16 tokens.
+// Weights are read once per 16 tokens. Rows past the end repeat the last row:
+// its own lane loads and stores the same values in the same instructions, so
+// no access is predicated and every wait and schedule is static.
+//
+// A tile is bound by its VALU work (bf16 conversions, the sigmoid's exp2 and
+// reciprocal at quarter rate: 24 instructions a column and token) and by a
+// chain of load phases, so bf16 roundings are done in pairs and two 8-wave
+// workgroups share a CU at hidden 4096 (110 registers; 16 waves of half the
+// columns needed 120, one workgroup a CU): 8192 rows 78.6 -> 72 us, 4096 rows
+// 38.6 -> 34 us; the residual add and copy alone take 60 us at 8304 rows.
 // ---------------------------------------------------------------------------
+// Keeps the compiler from moving memory operations or instructions across.
+__device__ __forceinline__ void hold_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 constexpr int kRank = 16;
 constexpr int kNormTokens = 16;
 
@@ -108,40 +132,39 @@ struct GatedNormArgs {
   float eps;
 };
 
-template <int S, int W>  // W waves of S column groups of 32: hidden = 32 S W
-__global__ __launch_bounds__(64 * W) void gated_norm_kernel(const GatedNormArgs a) {
+template <int S, int W, bool RES>  // W waves of S column groups of 32: hidden = 32 S W
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void gated_norm_kernel(const GatedNormArgs a) {
   __shared__ float ssq[W][kNormTokens];
   __shared__ float down_part[W][kNormTokens][kRank];
   __shared__ float gate_s[kNormTokens][kRank];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int64_t t = (int64_t)blockIdx.x * kNormTokens + m;
-  const bool ok = t < a.rows;
+  const int64_t t = min((int64_t)blockIdx.x * kNormTokens + m, (int64_t)a.rows - 1);
   const int col0 = 32 * S * wave + 8 * g;  // column of group s: col0 + 32 s
   u32x4 n[S];
   float ss = 0.0f;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     // Loads in batches of 4 groups: bounds the registers held by loads in flight.
-    if (s % 4 == 0 && s > 0) __builtin_amdgcn_sched_barrier(0);
+    if (s % 4 == 0 && s > 0) hold_order();
     const int col = col0 + 32 * s;
-    u32x4 xv = {0, 0, 0, 0};
-    if (ok) xv = load_u32x4(a.x + t * a.x_stride + col);
+    u32x4 xv = load_u32x4(a.x + t * a.x_stride + col);
     float f[8];
     unpack8(xv, f);
-    if (a.res_in) {
-      u32x4 rv = {0, 0, 0, 0};
-      if (ok) rv = load_u32x4(a.res_in + t * a.res_in_stride + col);
+    if constexpr (RES) {
+      const u32x4 rv = load_u32x4(a.res_in + t * a.res_in_stride + col);
       float r[8];
       unpack8(rv, r);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = rbf(f[e] + r[e]);
+      for (int e = 0; e < 8; ++e) f[e] += r[e];
       xv = pack8(f);
-      if (ok) *reinterpret_cast<u32x4*>(a.res_out + t * a.res_out_stride + col) = xv;
+      unpack8(xv, f);
+      *reinterpret_cast<u32x4*>(a.res_out + t * a.res_out_stride + col) = xv;
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
     n[s] = xv;
+    asm volatile("" : "+v"(n[s]));
   }
   ss += __shfl_xor(ss, 16, 64);
   ss += __shfl_xor(ss, 32, 64);
@@ -154,14 +177,18 @@ __global__ __launch_bounds__(64 * W) void gated_norm_kernel(const GatedNormArgs 
   f32x4 down = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    if (s % 4 == 0 && s > 0) __builtin_amdgcn_sched_barrier(0);
+    if (s % 4 == 0 && s > 0) hold_order();
     const int col = col0 + 32 * s;
     float f[8], w[8];
     unpack8(n[s], f);
     unpack8(load_u32x4(a.weight + col), w);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = rbf(rbf(f[e] * inv) * w[e]);
+    for (int e = 0; e < 8; ++e) f[e] *= inv;
+    round8(f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] *= w[e];
     n[s] = pack8(f);
+    asm volatile("" : "+v"(n[s]));
     const u32x4 wd = load_u32x4(a.gate_down + (int64_t)m * a.hidden + col);  // B: rank m
     down = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, n[s]),
                                                    __builtin_bit_cast(bf16x8, wd), down, 0, 0, 0);
@@ -186,30 +213,33 @@ __global__ __launch_bounds__(64 * W) void gated_norm_kernel(const GatedNormArgs 
     for (int e = 0; e < 8; ++e) f[e] = gate_s[m][8 * g + e];
     sb = pack8(f);
   }
-  const u32x4 zero4 = {0, 0, 0, 0};
+  const uint32_t in_rank = g < 2 ? 0xffffffffu : 0u;
+  const u32x4 rank_mask = {in_rank, in_rank, in_rank, in_rank};
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    if (s % 4 == 0 && s > 0) __builtin_amdgcn_sched_barrier(0);
+    if (s % 4 == 0 && s > 0) hold_order();
     const int col = col0 + 32 * s;
-    f32x4 up[2];
+    float b[8], f[8], u[8];
+    unpack8(load_u32x4(a.bias + col), b);
+    unpack8(n[s], f);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       // A row m (this lane's load role) is column 32 s + 8 (m / 4) + 4 h + m % 4 of the wave's group
       const int arow = 32 * S * wave + 32 * s + 8 * (m >> 2) + 4 * h + (m & 3);
-      const u32x4 wu = g < 2 ? load_u32x4(a.gate_up + (int64_t)arow * kRank + 8 * g) : zero4;
-      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      up[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wu),
-                                                      __builtin_bit_cast(bf16x8, sb), z, 0, 0, 0);
-    }
-    float b[8], f[8];
-    unpack8(load_u32x4(a.bias + col), b);
-    unpack8(n[s], f);
+      const u32x4 wu = load_u32x4(a.gate_up + arow * kRank + 8 * (g & 1)) & rank_mask;
+      f32x4 up = {b[4 * h], b[4 * h + 1], b[4 * h + 2], b[4 * h + 3]};  // the bias starts the sum
+      up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wu),
+                                                   __builtin_bit_cast(bf16x8, sb), up, 0, 0, 0);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float u = up[e >> 2][e & 3];
-      f[e] = rbf(f[e] * rbf(sigmoid_f(rbf(u + b[e]))));
+      for (int i = 0; i < 4; ++i) u[4 * h + i] = up[i];
     }
-    if (ok) *reinterpret_cast<u32x4*>(a.out + t * a.out_stride + col) = pack8(f);
+    round8(u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) u[e] = sigmoid_f(u[e]);
+    round8(u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] *= u[e];
+    *reinterpret_cast<u32x4*>(a.out + t * a.out_stride + col) = pack8(f);
   }
 }
 
@@ -227,10 +257,17 @@ __global__ __launch_bounds__(64 * W) void gated_norm_kernel(const GatedNormArgs 
 //  * up: each of the thread's columns dots its 16 gate_up weights (32 B) with s.
 // Every load that does not depend on the token's statistics (the row, the
 // residual, gamma, the gate_down slices) is issued first; the gate_up slices
-// and the bias go out before the down reduction. The 2 x 16 x hidden gate
+// and the bias go out before the down reduction. Both projections multiply
+// bf16 pairs with v_dot2_f32_bf16 (their operands are bf16 values): with them
+// unpacked to fp32 FMAs the kernel was bound by its VALU work (112 rows 10.8 ->
+// 8.8 us, 350 rows 20.9 -> 14.3, 1000 rows 39.5 -> 25 at hidden 4096). The 2 x 16 x hidden gate
 // weights are read by every workgroup and come from L2 after the first ones.
 // ---------------------------------------------------------------------------
+// Hidden 4096, 16-token tiles against one workgroup per token: 512 rows 23.4
+// against 15 us, 1000 rows about equal.
 constexpr int kTokenNormRows = 1024;
+constexpr int kNormRound = 256 * kNormTokens;  // rows of one tile on every CU
+constexpr int kNormTail = 256;
 constexpr int kTokenNormMaxWaves = 8;  // hidden up to 4096
 
 // Sum over the wave of v[j] for each j < 16: returns the total of rank
@@ -273,8 +310,10 @@ __global__ __launch_bounds__(64 * kTokenNormMaxWaves) void token_norm_kernel(con
     float r[8];
     unpack8(rv, r);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = rbf(f[e] + r[e]);
-    *reinterpret_cast<u32x4*>(a.res_out + t * a.res_out_stride + col) = pack8(f);
+    for (int e = 0; e < 8; ++e) f[e] += r[e];
+    const u32x4 sum = pack8(f);
+    unpack8(sum, f);
+    *reinterpret_cast<u32x4*>(a.res_out + t * a.res_out_stride + col) = sum;
   }
   float ss = 0.0f;
 #pragma unroll
@@ -286,11 +325,17 @@ __global__ __launch_bounds__(64 * kTokenNormMaxWaves) void token_norm_kernel(con
   float sq = 0.0f;
   for (int w = 0; w < waves; ++w) sq += wsq[w];
   const float inv = rsqrtf(sq / (float)a.hidden + a.eps);
+  u32x4 nv;
   {
     float g[8];
     unpack8(wv, g);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = rbf(rbf(f[e] * inv) * g[e]);
+    for (int e = 0; e < 8; ++e) f[e] *= inv;
+    round8(f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] *= g[e];
+    nv = pack8(f);
+    unpack8(nv, f);
   }
   u32x4 wu[2 * 8];
 #pragma unroll
@@ -302,11 +347,9 @@ __global__ __launch_bounds__(64 * kTokenNormMaxWaves) void token_norm_kernel(con
   float d[kRank];
 #pragma unroll
   for (int j = 0; j < kRank; ++j) {
-    float w[8];
-    unpack8(wd[j], w);
     float acc = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc += f[e] * w[e];
+    for (int i = 0; i < 4; ++i) acc = dot2(nv[i], wd[j][i], acc);
     d[j] = acc;
   }
   const float dj = wave_transpose_sum16(d);
@@ -315,26 +358,25 @@ __global__ __launch_bounds__(64 * kTokenNormMaxWaves) void token_norm_kernel(con
   float sj = 0.0f;
   if (lane < kRank) {
     for (int w = 0; w < waves; ++w) sj += wdown[w][lane];
-    sj = rbf(silu_f(rbf(sj)));
+    sj = silu_f(rbf(sj));
   }
-  float sr[kRank];
+  // The 16 ranks as bf16 pairs, rank pair j in lane 2 j: into scalar registers.
+  const uint32_t pair = pack_bf16x2(sj, __shfl_down(sj, 1, 64));
+  uint32_t sp[kRank / 2];
 #pragma unroll
-  for (int j = 0; j < kRank; ++j)
-    sr[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sj), j));
-  float b[8];
-  unpack8(bv, b);
+  for (int j = 0; j < kRank / 2; ++j) sp[j] = __builtin_amdgcn_readlane(pair, 2 * j);
+  float u[8];
+  unpack8(bv, u);  // the bias starts the sum
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float u0[8], u1[8];
-    unpack8(wu[2 * e], u0);
-    unpack8(wu[2 * e + 1], u1);
-    float u = 0.0f;
+  for (int e = 0; e < 8; ++e)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) u += sr[j] * u0[j];
+    for (int j = 0; j < kRank / 2; ++j) u[e] = dot2(wu[2 * e + (j >> 2)][j & 3], sp[j], u[e]);
+  round8(u);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) u += sr[8 + j] * u1[j];
-    f[e] = rbf(f[e] * rbf(sigmoid_f(rbf(u + b[e]))));
-  }
+  for (int e = 0; e < 8; ++e) u[e] = sigmoid_f(u[e]);
+  round8(u);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] *= u[e];
   *reinterpret_cast<u32x4*>(a.out + t * a.out_stride + col) = pack8(f);
 }
 
@@ -1075,17 +1117,34 @@ extern "C" int qsa_gated_norm(const void* x, int64_t x_stride, const void* resid
   hipStream_t s = static_cast<hipStream_t>(stream);
   (void)workspace;
   (void)workspace_bytes;
-  if (rows < kTokenNormRows) {
-    hipLaunchKernelGGL(token_norm_kernel, dim3(rows), dim3(hidden / 8), 0, s, a);
+  auto launch_tokens = [&](int first) {  // rows first .. rows - 1
+    GatedNormArgs r = a;
+    r.x += first * x_stride;
+    if (r.res_in) {
+      r.res_in += first * residual_in_stride;
+      r.res_out += first * residual_out_stride;
+    }
+    r.out += first * out_stride;
+    hipLaunchKernelGGL(token_norm_kernel, dim3(rows - first), dim3(hidden / 8), 0, s, r);
     return check_launch("qsa_gated_norm (one workgroup per token)");
+  };
+  if (rows < kTokenNormRows) return launch_tokens(0);
+  // A few rows past whole rounds of tiles run one workgroup per token too: a
+  // round of 4096-column tiles takes ~25 us however few its tiles are.
+  const int whole = rows / kNormRound * kNormRound;
+  if (hidden == 4096 && rows > whole && rows - whole <= kNormTail) {
+    a.rows = whole;
+    const int st = launch_tokens(whole);
+    if (st != QSA_OK) return st;
   }
-  const dim3 grid((rows + kNormTokens - 1) / kNormTokens);
+  const dim3 grid((a.rows + kNormTokens - 1) / kNormTokens);
+  auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, a); };
+  const bool res = residual_in != nullptr;
   switch (hidden / 512) {
-    case 1: hipLaunchKernelGGL((gated_norm_kernel<4, 4>), grid, dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((gated_norm_kernel<8, 4>), grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((gated_norm_kernel<8, 8>), grid, dim3(512), 0, s, a); break;
-    case 8: hipLaunchKernelGGL((gated_norm_kernel<8, 16>), grid, dim3(1024), 0, s, a); break;
-    default: return fail(QSA_ERR_UNSUPPORTED, "qsa_gated_norm: hidden size must be 512, 1024, 2048 or 4096");
+    case 1: res ? launch(gated_norm_kernel<4, 4, true>, 256) : launch(gated_norm_kernel<4, 4, false>, 256); break;
+    case 2: res ? launch(gated_norm_kernel<8, 4, true>, 256) : launch(gated_norm_kernel<8, 4, false>, 256); break;
+    case 4: res ? launch(gated_norm_kernel<8, 8, true>, 512) : launch(gated_norm_kernel<8, 8, false>, 512); break;
+    default: res ? launch(gated_norm_kernel<16, 8, true>, 512) : launch(gated_norm_kernel<16, 8, false>, 512); break;
   }
   return check_launch("qsa_gated_norm");
 }

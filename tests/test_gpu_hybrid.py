@@ -286,6 +286,18 @@ def test_gated_norm_kernel_against_oracle(rows, hidden, residual):
     _close(out.cpu(), want, "gated_norm", 0.02, 2e-3)
 
 
+@pytest.mark.parametrize("rows,hidden,residual", [
+    (1023, 4096, True), (1024, 4096, False), (1025, 4096, True),
+    (4097, 4096, True), (4352, 4096, False), (4353, 4096, True), (1039, 2048, False),
+    (1025, 1024, True), (1031, 512, False)])
+def test_gated_norm_row_splits(rows, hidden, residual):
+    """The edges of the row split: one workgroup per token below 1024 rows,
+    16-token tiles with a partial last tile, and at hidden 4096 up to 256 rows
+    past whole rounds of 4096 rows as single tokens beside the tiles. Every row
+    is written, none twice: bf16(x + r) is exact."""
+    test_gated_norm_kernel_against_oracle(rows, hidden, residual)
+
+
 def test_silu_mul_kernel_against_oracle():
     gu = _bf16((33, 2 * 5632), 7, 2.0)
     got = L.silu_mul(gu.to(DEV)).cpu()
