@@ -31,7 +31,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .ops.indexer import _visible_blocks, decode_select_attend
+from .ops.indexer import _visible_blocks, decode_layer
 from .ops.indexer import select_paged_tokens as qsa_select_paged_tokens  # attention.py:21
 from .ops.normalization import IndexerRMSNorm, rotary_cache
 from .ops.prepare import qsa_prepare
@@ -144,6 +144,22 @@ def main_kv_views(kv_cache: torch.Tensor, head_size: int) -> tuple[torch.Tensor,
     physical layouts backs it (``backend.py:100-102``); ``backend.py:148-153``
     swaps the head and page dims and splits the last one.
     """
+    if kv_cache.dim() == 4 and kv_cache.size(3) == 2 * head_size:
+        # Both views at once: a decode step asks for them on every call.
+        blocks, heads, page, _ = kv_cache.shape
+        s_block, s_head, s_page, s_dim = kv_cache.stride()
+        if head_size == 1:
+            s_dim = 1
+        if heads == 1:
+            s_head = s_dim * head_size
+        if page == 1:
+            s_page = s_head * heads
+        if blocks == 1:
+            s_block = s_page * page
+        shape, strides = (blocks, page, heads, head_size), (s_block, s_page, s_head, s_dim)
+        first = kv_cache.storage_offset()
+        return (kv_cache.as_strided(shape, strides, first),
+                kv_cache.as_strided(shape, strides, first + head_size * kv_cache.stride(3)))
     key_cache, value_cache = kv_cache.transpose(1, 2).split(head_size, dim=-1)
     return (canonicalize_singleton_dim_strides(key_cache),
             canonicalize_singleton_dim_strides(value_cache))
@@ -235,19 +251,15 @@ def run_qsa(layer: QSALayerState, impl: YuLanQSAImpl, index_query: torch.Tensor,
         # One token per request: scoring, then the top-k + expansion and the
         # attention as one op (the same selection into the layer's buffers and
         # the same output as the two calls below).
-        t2r = compressed.token_to_req[:count]
-        pos = compressed.logical_positions[:count]
         visible = compressed.visible_blocks
-        visible = (visible[:count] if visible is not None
-                   else _visible_blocks(pos, compressed.seq_lens, t2r, compress_ratio))
-        output[count:].zero_()
-        decode_select_attend(
-            index_query[:count], compressed_key_cache, compressed.block_table, visible,
-            query[:count], key_cache, value_cache, main.block_table, t2r, pos,
-            compressed.seq_lens, token_topk,
-            compress_ratio, compressed.max_seq_len, layer.topk_indices_buffer[:count],
-            layer.topk_counts_buffer[:count], output[:count],
-            output_gate=gate[:count] if gate is not None else None)
+        if visible is None:
+            visible = _visible_blocks(compressed.logical_positions[:count], compressed.seq_lens,
+                                      compressed.token_to_req[:count], compress_ratio)
+        decode_layer(
+            index_query, compressed_key_cache, compressed.block_table, visible, query, key_cache,
+            value_cache, main.block_table, compressed.token_to_req, compressed.logical_positions,
+            compressed.seq_lens, count, token_topk, compress_ratio, compressed.max_seq_len,
+            layer.topk_indices_buffer, layer.topk_counts_buffer, output, gate)
         return output
     select_for_layer(
         index_query[:count], compressed_key_cache, compressed,

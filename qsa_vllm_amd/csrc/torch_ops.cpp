@@ -507,6 +507,35 @@ void decode_select_attend_impl(const Tensor& scores, const Tensor& lengths, cons
         "qsa_decode_select_attention");
 }
 
+// A uniform one-token decode batch of one layer, scoring to attention output:
+// the rows are the first `count` of each per-row tensor, the output's rows
+// past them are zeroed. One dispatcher call: an eager decode step of few rows
+// is bound by the host's work per call, and as separate slices, a logits
+// allocation and two ops this took 31 us a step (one row) against ~20 us here.
+void decode_layer_impl(const Tensor& index_q, const Tensor& index_cache, const Tensor& index_table,
+                       const Tensor& visible, const Tensor& q, const Tensor& k_cache,
+                       const Tensor& v_cache, const Tensor& table, const Tensor& token_to_req,
+                       const Tensor& pos, const Tensor& sequence_lengths, int64_t count,
+                       int64_t columns, int64_t ratio, const Tensor& indices, const Tensor& counts,
+                       const Tensor& out, const OptTensor& output_gate) {
+  QSA_REQUIRE(count >= 0 && columns > 0, "count must not be negative, columns must be positive");
+  const auto head = [count](const Tensor& t) {
+    return t.size(0) <= count ? t : t.narrow(0, 0, count);
+  };
+  for (const Tensor* t : {&index_q, &visible, &q, &token_to_req, &pos, &indices, &counts, &out})
+    QSA_REQUIRE(t->dim() > 0, "per-row tensors must have rows");
+  if (out.size(0) > count) out.narrow(0, count, out.size(0) - count).zero_();
+  const Tensor iq = head(index_q), vis = head(visible);
+  if (iq.size(0) == 0) return;
+  const Tensor logits = at::empty({iq.size(0), columns}, iq.options().dtype(at::kFloat));
+  indexer_decode_impl(iq, index_cache, index_table, vis, logits, 1);
+  OptTensor gate;
+  if (output_gate.has_value() && output_gate->defined()) gate = head(*output_gate);
+  decode_select_attend_impl(logits, vis, head(pos), sequence_lengths, head(token_to_req), table,
+                            head(indices), head(counts), ratio, head(q), k_cache, v_cache,
+                            head(out), gate, 0);
+}
+
 void sparse_attention_merge_impl(const Tensor& partial_out, const Tensor& partial_lse,
                                  const Tensor& out, const OptTensor& output_gate) {
   const auto dev = on_gpu({&partial_out, &partial_lse, &out, opt(output_gate)});
@@ -818,6 +847,11 @@ TORCH_LIBRARY_FRAGMENT(yulan_qsa_kernels, m) {
       "Tensor sequence_lengths, Tensor token_to_req, Tensor table, Tensor(a!) indices, "
       "Tensor(b!) counts, int ratio, Tensor q, Tensor k_cache, Tensor v_cache, Tensor(c!) out, "
       "Tensor? output_gate, int num_splits) -> ()");
+  m.def(
+      "decode_layer(Tensor index_q, Tensor index_cache, Tensor index_table, Tensor visible, "
+      "Tensor q, Tensor k_cache, Tensor v_cache, Tensor table, Tensor token_to_req, "
+      "Tensor positions, Tensor sequence_lengths, int count, int columns, int ratio, "
+      "Tensor(a!) indices, Tensor(b!) counts, Tensor(c!) out, Tensor? output_gate) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(yulan_qsa_kernels, CUDA, m) {
@@ -835,6 +869,7 @@ TORCH_LIBRARY_IMPL(yulan_qsa_kernels, CUDA, m) {
   m.impl("sparse_attention", &sparse_attention_impl);
   m.impl("sparse_attention_merge", &sparse_attention_merge_impl);
   m.impl("decode_select_attend", &decode_select_attend_impl);
+  m.impl("decode_layer", &decode_layer_impl);
 }
 
 // Shape-only tracing (fake / meta tensors): the ops mutate their outputs in
@@ -865,6 +900,11 @@ TORCH_LIBRARY_IMPL(yulan_qsa_kernels, Meta, m) {
          [](const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
             const Tensor&, const Tensor&, const Tensor&, int64_t, const Tensor&, const Tensor&,
             const Tensor&, const Tensor&, const OptTensor&, int64_t) {});
+  m.impl("decode_layer",
+         [](const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+            const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+            const Tensor&, int64_t, int64_t, int64_t, const Tensor&, const Tensor&, const Tensor&,
+            const OptTensor&) {});
   m.impl("indexer_prepare",
          [](const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, double,
             const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,

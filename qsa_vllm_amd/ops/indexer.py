@@ -108,6 +108,30 @@ def decode_select_attend(
     return out
 
 
+def decode_layer(index_q, index_cache, index_table, visible_blocks, q, k_cache, v_cache,
+                 main_block_table, token_to_req, query_positions, sequence_lengths, count,
+                 token_topk, compress_ratio, max_seq_len, indices_out, counts_out, out,
+                 output_gate) -> None:
+    """:func:`decode_select_attend` on the first ``count`` rows of every per-row
+    tensor, with the rows of ``out`` past them zeroed; one op call when the
+    logits fit the workspace cap."""
+    columns = decode_logits_columns(max_seq_len, compress_ratio,
+                                    index_table.shape[1] * index_cache.shape[1])
+    if columns > 0 and count * columns * 4 <= _LOGITS_CAP_BYTES:
+        torch.ops.yulan_qsa_kernels.decode_layer(
+            index_q, index_cache, index_table, visible_blocks, q, k_cache, v_cache,
+            main_block_table, token_to_req, query_positions, sequence_lengths, count, columns,
+            compress_ratio, indices_out, counts_out, out, output_gate)
+        return
+    out[count:].zero_()
+    decode_select_attend(
+        index_q[:count], index_cache, index_table, visible_blocks[:count], q[:count], k_cache,
+        v_cache, main_block_table, token_to_req[:count], query_positions[:count],
+        sequence_lengths, token_topk, compress_ratio, max_seq_len, indices_out[:count],
+        counts_out[:count], out[:count],
+        output_gate=output_gate[:count] if output_gate is not None else None)
+
+
 def qsa_select_paged_prefill(
     q: torch.Tensor,
     k_cache: torch.Tensor,

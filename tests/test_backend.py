@@ -41,6 +41,30 @@ def test_main_kv_views_address_the_bound_cache(heads, layout):
         assert k.stride(2) == d          # canonical stride of the singleton head dim
 
 
+@pytest.mark.parametrize("shape,head_size", [
+    ((5, 2, 16, 256), 128), ((1, 2, 16, 256), 128), ((5, 1, 16, 256), 128), ((5, 2, 1, 256), 128),
+    ((1, 1, 1, 8), 4), ((3, 1, 1, 2), 1), ((1, 3, 2, 2), 1), ((0, 2, 16, 64), 32)])
+@pytest.mark.parametrize("layout", ["head_major", "token_major", "offset", "strided"])
+def test_main_kv_views_equal_the_general_form(shape, head_size, layout):
+    """Shape, strides and address of both views, for every singleton dim and
+    physical order, as transpose + split + canonical singleton strides give them."""
+    backend = _backend()
+    b, h, p, w = shape
+    if layout == "token_major":
+        kv = torch.zeros(b, p, h, w).permute(0, 2, 1, 3)
+    elif layout == "offset":
+        kv = torch.zeros(b + 2, h, p, w)[2:]
+    elif layout == "strided":
+        kv = torch.zeros(2 * b, h, p, 2 * w)[::2, :, :, ::2]
+    else:
+        kv = torch.zeros(shape)
+    for got, part in zip(backend.main_kv_views(kv, head_size),
+                         kv.transpose(1, 2).split(head_size, dim=-1)):
+        want = backend.canonicalize_singleton_dim_strides(part)
+        assert got.shape == want.shape and got.stride() == want.stride()
+        assert got.storage_offset() == want.storage_offset()
+
+
 def test_canonical_strides_keep_addresses():
     backend = _backend()
     base = torch.arange(2 * 1 * 5 * 1 * 4, dtype=torch.float32).view(2, 5, 4)
@@ -131,6 +155,21 @@ def _expected_selection(wl, physical):
         idx.append(i)
         cnt.append(c)
     return torch.cat(idx), torch.cat(cnt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pad_rows", [0, 3])
+def test_run_qsa_uniform_decode_past_the_logits_cap(monkeypatch, pad_rows):
+    """One op call or, when the logits exceed the workspace cap, the span-wise
+    selection and the attention: the same selection and output."""
+    from qsa_vllm_amd.ops import indexer
+    wl = make_workload("cpu_decode_4k", device=DEV, batch=5, gate=True)
+    print(f"[backend] uniform decode, logits cap, pad {pad_rows}", flush=True)
+    layer, output = _run_layer(wl, pad_rows)
+    monkeypatch.setattr(indexer, "_LOGITS_CAP_BYTES", 4 * 512)
+    capped_layer, capped = _run_layer(wl, pad_rows)
+    assert torch.equal(layer.topk_indices_buffer[:5], capped_layer.topk_indices_buffer[:5])
+    assert torch.equal(output, capped)
 
 
 @pytest.mark.gpu
