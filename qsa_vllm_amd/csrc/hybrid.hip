@@ -30,6 +30,8 @@
 // per key head); the conv channels are ordered [q of all key heads, k of all
 // key heads, v of all value heads]; conv state [slots, K-1, channels] bf16
 // (oldest row first); recurrent state [slots, value heads, 128, 128] fp32.
+#include <type_traits>
+
 #include "gdn_args.h"
 #include "../../include/qsa_hip.h"
 
@@ -442,101 +444,132 @@ struct GdnPrepArgs {
   uint16_t* v_out;  // [tokens, value_heads, 128]
   float* g_out;     // [tokens, value_heads]
   float* beta_out;
+  bool conv_w_aligned;  // 16 bytes
 };
 
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
-// One token per workgroup; thread i covers channels 16 i .. 16 i + 15.
-template <int K>
-__global__ __launch_bounds__(1024) void gdn_prep_kernel(const GdnPrepArgs a) {
-  const int t = blockIdx.x;
+// TT consecutive tokens and 2048 channels per workgroup, 8 channels per thread.
+// The convolution's window slides over the tokens in registers, so a row is
+// read once (and K - 1 rows again per workgroup) and the weights once per TT
+// tokens. Taps before a token's sequence come from its conv state. Bound by
+// HBM: 8192 tokens of 4096 channels move 167 MB in 38 us (4.4 TB/s); one token
+// per workgroup with 16 channels a thread read each row four times at 4 waves a
+// SIMD and took 72 us.
+template <int K, int TT>
+__global__ __launch_bounds__(256) void gdn_prep_kernel(const GdnPrepArgs a) {
   const GdnShape& s = a.s;
-  // A token whose sequence entry is out of range, or whose range does not
+  const int lane = threadIdx.x & 63;
+  const int t0 = blockIdx.x * TT, nt = min(TT, a.tokens - t0);
+  // Lane i < TT: token t0 + i's offset in its sequence and its state slot. A
+  // token whose sequence entry is out of range, or whose range does not
   // contain it, is treated as the first token of a sequence without state.
-  const int seq_raw = a.token_seq[t];
-  const bool seq_ok = seq_raw >= 0 && seq_raw < a.num_seqs;
-  const int seq = seq_ok ? seq_raw : 0;
-  int start = seq_ok ? a.seq_start[seq] : t;
-  int64_t slot = seq_ok ? a.slots[seq] : -1;
-  if (start < 0 || start > t) {
-    start = t;
-    slot = -1;
+  int off_l, slot_l;
+  {
+    const int t = t0 + min(lane, nt - 1);
+    const int seq_raw = a.token_seq[t];
+    const bool seq_ok = seq_raw >= 0 && seq_raw < a.num_seqs;
+    const int seq = seq_ok ? seq_raw : 0;
+    int start = seq_ok ? a.seq_start[seq] : t;
+    int64_t slot = seq_ok ? a.slots[seq] : -1;
+    if (start < 0 || start > t) {
+      start = t;
+      slot = -1;
+    }
+    off_l = t - start;
+    slot_l = slot >= 0 && slot < a.num_slots ? (int)slot : -1;
   }
-  const int off = t - start;
-  const bool slot_ok = slot >= 0 && slot < a.num_slots;
-  const int c0 = 16 * threadIdx.x;
-  const bool active = c0 < s.channels;
-  float acc[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+  const int c0 = 8 * (blockIdx.y * 256 + threadIdx.x);
+  const bool active = c0 < s.channels;  // whole heads (16 threads) are active or not
   if (active) {
-    const int col = gdn_column(c0, s);
-    // weights: 16 channels x K taps, channel-major (16 K contiguous bf16)
-    float w[16][K];
+    const uint16_t* column = a.qkvz + gdn_column(c0, s);
+    u32x4 x[TT + K - 1];  // rows t0 - (K - 1) .. t0 + TT - 1
+#pragma unroll
+    for (int i = 0; i < TT + K - 1; ++i) {
+      const int row = min(max(t0 - (K - 1) + i, 0), a.tokens - 1);
+      if (TT > 1 || i == K - 1) x[i] = load_u32x4(column + (int64_t)row * a.qkvz_stride);
+    }
+    float w[8][K];  // 8 channels x K taps, channel-major (8 K contiguous bf16)
     const uint16_t* wp = a.conv_w + (int64_t)c0 * K;
+    if (a.conv_w_aligned) {
+      u32x4 wv[K];
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
+      for (int i = 0; i < K; ++i) wv[i] = load_u32x4(wp + 8 * i);
 #pragma unroll
-      for (int j = 0; j < K; ++j) w[e][j] = __builtin_bit_cast(float, (uint32_t)wp[e * K + j] << 16);
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      const int src = off - (K - 1) + j;
-      const uint16_t* row;
-      bool ok = true;
-      if (src >= 0) {
-        row = a.qkvz + (int64_t)(start + src) * a.qkvz_stride + col;
-      } else {
-        ok = slot_ok;
-        row = a.conv_state + (slot_ok ? (slot * (K - 1) + (K - 1 + src)) * s.channels + c0 : 0);
-      }
-      float x[16] = {};
-      if (ok) {
-        unpack8(load_u32x4(row), *reinterpret_cast<float(*)[8]>(&x[0]));
-        unpack8(load_u32x4(row + 8), *reinterpret_cast<float(*)[8]>(&x[8]));
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] += w[e][j] * x[e];
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = rbf(silu_f(acc[e]));
-  }
-  // l2 norm over each 128-channel q/k head: 8 consecutive threads.
-  const int qk = s.key_heads * kHeadDim;
-  float ss = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) ss += acc[e] * acc[e];
-  ss += __shfl_xor(ss, 1, 64);
-  ss += __shfl_xor(ss, 2, 64);
-  ss += __shfl_xor(ss, 4, 64);
-  if (active) {
-    if (c0 < 2 * qk) {
-      const bool is_q = c0 < qk;
-      const int cc = is_q ? c0 : c0 - qk;
-      const float inv = rsqrtf(ss + 1e-6f);
-      const float scale = is_q ? rsqrtf((float)kHeadDim) : 1.0f;
-      float* dst = (is_q ? a.q_out : a.k_out) + ((int64_t)t * s.key_heads) * kHeadDim + cc;
-#pragma unroll
-      for (int e = 0; e < 16; e += 4) {
-        f32x4 v;
-        v[0] = acc[e] * inv * scale;
-        v[1] = acc[e + 1] * inv * scale;
-        v[2] = acc[e + 2] * inv * scale;
-        v[3] = acc[e + 3] * inv * scale;
-        *reinterpret_cast<f32x4*>(dst + e) = v;
-      }
+      for (int i = 0; i < 8 * K; ++i)
+        w[i / K][i % K] = i & 1 ? bf16_hi(wv[i / 8][(i & 7) >> 1]) : bf16_lo(wv[i / 8][(i & 7) >> 1]);
     } else {
-      uint16_t* dst = a.v_out + (int64_t)t * s.value_heads * kHeadDim + (c0 - 2 * qk);
-      *reinterpret_cast<u32x4*>(dst) = pack8(*reinterpret_cast<float(*)[8]>(&acc[0]));
-      *reinterpret_cast<u32x4*>(dst + 8) = pack8(*reinterpret_cast<float(*)[8]>(&acc[8]));
+#pragma unroll
+      for (int i = 0; i < 8 * K; ++i) w[i / K][i % K] = bf16_lo(wp[i]);
+    }
+    const int qk = s.key_heads * kHeadDim;
+    float win[K][8];  // the last K rows, row t - (K - 1) + j in win[(i + j) % K]
+#pragma unroll
+    for (int i = 0; i < K - 1; ++i)
+      if (TT > 1) unpack8(x[i], win[i]);
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      if (i >= nt) break;
+      const int64_t t = t0 + i;
+      const int off = __builtin_amdgcn_readlane(off_l, i), slot = __builtin_amdgcn_readlane(slot_l, i);
+      unpack8(x[i + K - 1], win[(i + K - 1) % K]);
+      float acc[8] = {};
+      if (TT > 1 && off >= K - 1) {
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += w[e][j] * win[(i + j) % K][e];
+      } else {
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+          const int src = off - (K - 1) + j;
+          float tap[8] = {};
+          if (src >= 0) {
+            if (TT == 1 && j < K - 1) unpack8(load_u32x4(column + (t - (K - 1) + j) * a.qkvz_stride), tap);
+            else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) tap[e] = win[(i + j) % K][e];
+            }
+          } else if (slot >= 0) {
+            unpack8(load_u32x4(a.conv_state + ((int64_t)slot * (K - 1) + (K - 1 + src)) * s.channels + c0), tap);
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += w[e][j] * tap[e];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = silu_f(acc[e]);
+      const u32x4 rounded = pack8(acc);
+      if (c0 >= 2 * qk) {
+        *reinterpret_cast<u32x4*>(a.v_out + t * s.value_heads * kHeadDim + (c0 - 2 * qk)) = rounded;
+      } else {
+        // l2 norm over each 128-channel q/k head: 16 consecutive threads.
+        unpack8(rounded, acc);
+        float ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += acc[e] * acc[e];
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, 64);
+        const bool is_q = c0 < qk;
+        const float inv = rsqrtf(ss + 1e-6f);
+        const float scale = is_q ? rsqrtf((float)kHeadDim) : 1.0f;
+        float* dst = (is_q ? a.q_out + c0 : a.k_out + (c0 - qk)) + t * qk;
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<f32x4*>(dst + e) = f32x4{acc[e] * inv * scale, acc[e + 1] * inv * scale,
+                                                     acc[e + 2] * inv * scale, acc[e + 3] * inv * scale};
+      }
     }
   }
-  if ((int)threadIdx.x < s.value_heads) {
-    const int h = threadIdx.x, m = h / s.r, hl = h - m * s.r;
-    const uint16_t* bar = a.ba + (int64_t)t * a.ba_stride + m * 2 * s.r;
-    const float b = __builtin_bit_cast(float, (uint32_t)bar[hl] << 16);
-    const float av = __builtin_bit_cast(float, (uint32_t)bar[s.r + hl] << 16);
-    a.g_out[(int64_t)t * s.value_heads + h] = -expf(a.A_log[h]) * softplus_f(av + a.dt_bias[h]);
-    a.beta_out[(int64_t)t * s.value_heads + h] = sigmoid_f(b);
+  if (blockIdx.y == 0) {
+    for (int i = threadIdx.x; i < nt * s.value_heads; i += 256) {
+      const int64_t t = t0 + i / s.value_heads;
+      const int h = i % s.value_heads, m = h / s.r, hl = h - m * s.r;
+      const uint16_t* bar = a.ba + t * a.ba_stride + m * 2 * s.r;
+      const float b = bf16_lo(bar[hl]), av = bf16_lo(bar[s.r + hl]);
+      a.g_out[t * s.value_heads + h] = -expf(a.A_log[h]) * softplus_f(av + a.dt_bias[h]);
+      a.beta_out[t * s.value_heads + h] = sigmoid_f(b);
+    }
   }
 }
 
@@ -1186,13 +1219,27 @@ extern "C" int qsa_gdn_prep(const void* qkvz, int64_t qkvz_stride, const void* b
                 ba_stride, static_cast<const uint16_t*>(conv_weight),
                 static_cast<const uint16_t*>(conv_state), query_start_loc, token_to_seq, slots,
                 A_log, dt_bias, s, tokens, num_seqs, num_slots, q_out, k_out,
-                static_cast<uint16_t*>(v_out), g_out, beta_out};
-  const int threads = ((s.channels / 16 + 63) / 64) * 64;
+                static_cast<uint16_t*>(v_out), g_out, beta_out, aligned16(conv_weight)};
+  // Tokens per workgroup: more of them read less, fewer spread a small batch
+  // over the chip, and tokens at the start of a sequence (decode) fetch conv
+  // state instead of sharing rows. 4096 channels, 1 / 4 / 8 tokens, us: 256
+  // decode requests 4.9 / 7.9 / 12.3, a prompt of 600 tokens 7.3 / 7.4 / 9.4,
+  // 1024 11.2 / 8.4 / 10.1, 4096 33.5 / 23.4 / 22.3, 8192 61 / 40 / 38.
+  const int parts = (s.channels + 2047) / 2048;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto kernel, int tt) {
+    hipLaunchKernelGGL(kernel, dim3((tokens + tt - 1) / tt, parts), dim3(256), 0, st, a);
+  };
+  auto launch_tokens = [&](auto k) {
+    constexpr int K = decltype(k)::value;
+    if (tokens / 4 < num_seqs || (int64_t)tokens * parts < 2048) launch(gdn_prep_kernel<K, 1>, 1);
+    else if ((int64_t)tokens * parts < 8192) launch(gdn_prep_kernel<K, 4>, 4);
+    else launch(gdn_prep_kernel<K, 8>, 8);
+  };
   switch (conv_kernel) {
-    case 2: hipLaunchKernelGGL(gdn_prep_kernel<2>, dim3(tokens), dim3(threads), 0, st, a); break;
-    case 3: hipLaunchKernelGGL(gdn_prep_kernel<3>, dim3(tokens), dim3(threads), 0, st, a); break;
-    default: hipLaunchKernelGGL(gdn_prep_kernel<4>, dim3(tokens), dim3(threads), 0, st, a); break;
+    case 2: launch_tokens(std::integral_constant<int, 2>()); break;
+    case 3: launch_tokens(std::integral_constant<int, 3>()); break;
+    default: launch_tokens(std::integral_constant<int, 4>()); break;
   }
   return check_launch("qsa_gdn_prep");
 }

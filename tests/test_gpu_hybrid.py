@@ -584,3 +584,55 @@ def test_gdn_recurrence_chunk_edges(hk, hv, lens, bound):
             _close(state[slot].cpu(), want_s, f"state, sequence of {m}", 1e-2, 1e-3)
     for slot in untouched:
         assert torch.equal(state[slot].cpu(), state0[slot])
+
+
+@pytest.mark.parametrize("K,hk,hv,lens,shift", [
+    (4, 2, 4, [1, 1, 2, 3, 1, 5, 4], 0),                       # one token per workgroup
+    (4, 2, 4, [3, 1000, 1, 2, 1042], 0),                       # four
+    (4, 2, 4, [2, 4093, 1, 4, 4101], 1),                       # eight; weights off 16-byte alignment
+    (4, 8, 16, [1022, 2], 0),                                  # two channel parts
+    (3, 2, 6, [2, 4097, 1, 4100], 0), (2, 1, 1, [1, 8200, 1], 1), (3, 2, 6, [5, 2], 1),
+])
+def test_gdn_prep_token_groups(K, hk, hv, lens, shift):
+    """Conv + SiLU, l2 norms and gates in every token grouping: sequence starts
+    inside a group, groups past the end, a sequence without a state slot, weights
+    at any alignment. fp32 arithmetic against float64 (bf16 rounding of v and of
+    the conv before the norm: 2^-8 relative, doubled)."""
+    gen = torch.Generator().manual_seed(sum(lens) + K)
+    channels, r, t, n = (2 * hk + hv) * 128, hv // hk, sum(lens), len(lens)
+    qkvz = torch.randn(t, hk * (2 + 2 * r) * 128, generator=gen).to(torch.bfloat16)
+    ba = torch.randn(t, 2 * hv, generator=gen).to(torch.bfloat16)
+    weight = (0.5 * torch.randn(channels, K, generator=gen)).to(torch.bfloat16)
+    conv = torch.randn(n + 1, K - 1, channels, generator=gen).to(torch.bfloat16)
+    A_log, dt_bias = torch.randn(hv, generator=gen), torch.randn(hv, generator=gen)
+    slots = torch.randperm(n + 1, generator=gen)[:n]
+    slots[n - 1] = -1
+    starts = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32)
+    seq = torch.repeat_interleave(torch.arange(n, dtype=torch.int32), torch.tensor(lens))
+    print(f"[hybrid] gdn prep K={K} heads {hk}/{hv} {lens} shift {shift}", flush=True)
+    flat = torch.zeros(channels * K + 8, dtype=torch.bfloat16, device=DEV)
+    w_dev = flat[shift:shift + channels * K].view(channels, K)
+    w_dev.copy_(weight)
+    q, k, v, g, beta = L.gdn_prep(qkvz.to(DEV), ba.to(DEV), w_dev, conv.to(DEV), starts.to(DEV),
+                                  seq.to(DEV), slots.to(DEV), A_log.to(DEV), dt_bias.to(DEV), hk, hv)
+    torch.cuda.synchronize()
+    x = qkvz.double().view(t, hk, (2 + 2 * r) * 128)
+    parts = x.split((128, 128, r * 128, r * 128), -1)
+    mixed = torch.cat([p.reshape(t, -1) for p in parts[:3]], -1)
+    out = torch.empty_like(mixed)
+    for i in range(n):
+        a, b = int(starts[i]), int(starts[i + 1])
+        old = conv[slots[i]].double() if slots[i] >= 0 else torch.zeros(K - 1, channels).double()
+        rows = torch.cat((old, mixed[a:b]))
+        out[a:b] = sum(weight[:, j].double() * rows[j:j + b - a] for j in range(K))
+    out = torch.nn.functional.silu(out)
+    wq, wk, wv = out.split((hk * 128, hk * 128, hv * 128), -1)
+    unit = lambda y: y * torch.rsqrt(y.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    wq, wk = unit(wq.view(t, hk, 128)) * 128 ** -0.5, unit(wk.view(t, hk, 128))
+    for got, want, name in ((q, wq, "q"), (k, wk, "k"), (v, wv.view(t, hv, 128), "v")):
+        # Each element's rounding is at most 2^-9 of it, so the mean is below 2^-9 of the largest.
+        _close(got.cpu(), want.float(), f"prep {name}", 2 ** -7, 2 ** -9)
+    bb, aa = ba.double().view(t, hk, 2 * r).split(r, -1)
+    want_g = -A_log.double().exp() * torch.nn.functional.softplus(aa.reshape(t, hv) + dt_bias.double())
+    _close(g.cpu(), want_g.float(), "prep g", 1e-5, 1e-6)
+    _close(beta.cpu(), torch.sigmoid(bb.reshape(t, hv)).float(), "prep beta", 1e-5, 1e-6)
