@@ -32,13 +32,11 @@
 // (oldest row first); recurrent state [slots, value heads, 128, 128] fp32.
 #include <type_traits>
 
-#include "gdn_args.h"
+#include "gdn_device.h"
 #include "../../include/qsa_hip.h"
 
 namespace qsa {
 namespace {
-
-constexpr int kHeadDim = 128;
 
 __device__ __forceinline__ float rbf(float x) { return bf16_lo(pack_bf16x2(x, 0.0f)); }
 // Sigmoid and SiLU through the hardware exp2 and reciprocal, each within a
@@ -50,14 +48,6 @@ __device__ __forceinline__ float sigmoid_f(float x) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
 __device__ __forceinline__ float silu_f(float x) { return x * sigmoid_f(x); }
-
-__device__ __forceinline__ void unpack8(const u32x4& v, float (&f)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = bf16_lo(v[i]);
-    f[2 * i + 1] = bf16_hi(v[i]);
-  }
-}
 
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
   u32x4 v;
@@ -613,97 +603,9 @@ __global__ __launch_bounds__(256) void gdn_conv_state_kernel(const GdnConvStateA
   }
 }
 
-constexpr int kRecTokens = 16;  // tokens staged in LDS per block
-
 __global__ __launch_bounds__(256) void gdn_recurrence_kernel(const GdnRecurArgs a) {
-  __shared__ float sq[kRecTokens][kHeadDim];
-  __shared__ float sk[kRecTokens][kHeadDim];
-  __shared__ float sv[kRecTokens][kHeadDim];
-  __shared__ float sg[kRecTokens], sb[kRecTokens];
-  const int h = blockIdx.x % a.value_heads;
-  const int seq = a.num_seqs - 1 - (int)(blockIdx.x / a.value_heads);  // longest (prefill) first
-  const int m = h / (a.value_heads / a.key_heads);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int j = 32 * wave + (lane & 31);
-  const int half = lane >> 5;
-  const int start = a.seq_start[seq], len = a.seq_start[seq + 1] - start;
-  if (len <= 0 || len >= a.chunk_min || start < 0 || start + len > a.tokens) return;
-  const int64_t slot = a.slots[seq];
-  const bool slot_ok = slot >= 0 && slot < a.num_slots;
-  float* sp = a.state + ((slot_ok ? slot : 0) * a.value_heads + h) * (int64_t)(kHeadDim * kHeadDim) +
-              (int64_t)(64 * half) * kHeadDim + j;
-  float S[64];
-#pragma unroll
-  for (int i = 0; i < 64; ++i) S[i] = slot_ok ? sp[(int64_t)i * kHeadDim] : 0.0f;
-  for (int b0 = 0; b0 < len; b0 += kRecTokens) {
-    const int nb = min(kRecTokens, len - b0);
-    // stage: thread -> (token tt = tid / 16, 8 dims at 8 (tid % 16))
-    {
-      const int tt = threadIdx.x >> 4, d0 = 8 * (threadIdx.x & 15);
-      if (tt < nb) {
-        const int64_t t = start + b0 + tt;
-        const float* qp = a.q + (t * a.key_heads + m) * kHeadDim + d0;
-        const float* kp = a.k + (t * a.key_heads + m) * kHeadDim + d0;
-        *reinterpret_cast<f32x4*>(&sq[tt][d0]) = *reinterpret_cast<const f32x4*>(qp);
-        *reinterpret_cast<f32x4*>(&sq[tt][d0 + 4]) = *reinterpret_cast<const f32x4*>(qp + 4);
-        *reinterpret_cast<f32x4*>(&sk[tt][d0]) = *reinterpret_cast<const f32x4*>(kp);
-        *reinterpret_cast<f32x4*>(&sk[tt][d0 + 4]) = *reinterpret_cast<const f32x4*>(kp + 4);
-        float vv[8];
-        unpack8(load_u32x4(a.v + (t * a.value_heads + h) * kHeadDim + d0), vv);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sv[tt][d0 + e] = vv[e];
-        if ((threadIdx.x & 15) == 0) {
-          sg[tt] = a.g[t * a.value_heads + h];
-          sb[tt] = a.beta[t * a.value_heads + h];
-        }
-      }
-    }
-    __syncthreads();
-    for (int tt = 0; tt < nb; ++tt) {
-      const float* kr = &sk[tt][64 * half];
-      float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, p3 = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 64; i += 4) {
-        const f32x4 kv = *reinterpret_cast<const f32x4*>(kr + i);
-        p0 += kv[0] * S[i];
-        p1 += kv[1] * S[i + 1];
-        p2 += kv[2] * S[i + 2];
-        p3 += kv[3] * S[i + 3];
-      }
-      const float ks = sum_wave_halves((p0 + p1) + (p2 + p3));
-      const float decay = expf(sg[tt]);
-      const float u = sb[tt] * (sv[tt][j] - decay * ks);
-#pragma unroll
-      for (int i = 0; i < 64; i += 4) {
-        const f32x4 kv = *reinterpret_cast<const f32x4*>(kr + i);
-        S[i] = S[i] * decay + kv[0] * u;
-        S[i + 1] = S[i + 1] * decay + kv[1] * u;
-        S[i + 2] = S[i + 2] * decay + kv[2] * u;
-        S[i + 3] = S[i + 3] * decay + kv[3] * u;
-      }
-      const float* qr = &sq[tt][64 * half];
-      p0 = p1 = p2 = p3 = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 64; i += 4) {
-        const f32x4 qv = *reinterpret_cast<const f32x4*>(qr + i);
-        p0 += qv[0] * S[i];
-        p1 += qv[1] * S[i + 1];
-        p2 += qv[2] * S[i + 2];
-        p3 += qv[3] * S[i + 3];
-      }
-      const float os = sum_wave_halves((p0 + p1) + (p2 + p3));
-      if (half == 0) {
-        const int64_t t = start + b0 + tt;
-        const __bf16 ob = (__bf16)os;
-        a.o[(t * a.value_heads + h) * kHeadDim + j] = __builtin_bit_cast(uint16_t, ob);
-      }
-    }
-    __syncthreads();
-  }
-  if (slot_ok) {
-#pragma unroll
-    for (int i = 0; i < 64; ++i) sp[(int64_t)i * kHeadDim] = S[i];
-  }
+  __shared__ GdnRecurLds L;
+  gdn_recurrence_block(a, blockIdx.x, L);
 }
 
 // ---------------------------------------------------------------------------
@@ -1301,16 +1203,15 @@ int gdn_recurrence(const float* q, const float* k, const void* v, const float* g
   if (chunks) {
     // Long sequences (chunks) first on the stream: their workgroups are the long ones.
     const size_t need = qsa_gdn_recurrence_workspace_bytes(tokens, num_seqs, key_heads, value_heads, max_seq_tokens);
-    int rc;
     if (workspace && need && aligned16(o)) {
       if (workspace_bytes < need || !aligned16(workspace))
         return fail(QSA_ERR_WORKSPACE, "qsa_gdn_recurrence: workspace too small or not 16-byte aligned");
-      rc = gdn_scan_launch(a, max_seq_tokens, workspace, st);
+      return gdn_scan_launch(a, max_seq_tokens, workspace, st);  // short sequences included
     } else {
       hipLaunchKernelGGL(gdn_chunk_kernel, dim3(num_seqs * value_heads), dim3(256), sizeof(ChunkLds), st, a);
-      rc = check_launch("qsa_gdn_recurrence (chunks)");
+      const int rc = check_launch("qsa_gdn_recurrence (chunks)");
+      if (rc != QSA_OK) return rc;
     }
-    if (rc != QSA_OK) return rc;
   }
   hipLaunchKernelGGL(gdn_recurrence_kernel, dim3(num_seqs * value_heads), dim3(256), 0, st, a);
   return check_launch("qsa_gdn_recurrence");
