@@ -16,7 +16,7 @@
 // The one-launch kernel (gdn_chunk_kernel) does all of it chunk after chunk in
 // one workgroup per (sequence, value head): ~14 us a chunk, and one prompt of
 // 8192 tokens kept 16 workgroups busy for 1812 us. Here it takes 44 us for the
-// operands (100 MB written, 67 MB of fp32 q and k read) and 117 us for the walk
+// operands (73 MB written, 67 MB of fp32 q and k read) and 117 us for the walk
 // (0.9 us a chunk, bound by the state waves' chain of products).
 #include "gdn_device.h"
 #include "../../include/qsa_hip.h"
@@ -276,7 +276,7 @@ __device__ __forceinline__ void chunk_operands(const GdnRecurArgs& a, uint16_t* 
 // One launch for the chunks' operands and the short sequences' per-token rule,
 // alternating, so that neither leaves the chip half empty at its end (112
 // decode requests beside 16 chunks of 512 tokens: 88 us against 48 + 42 as two
-// launches and the gap between them; together they move 405 MB, 4.6 TB/s).
+// launches and the gap between them; together they move 375 MB, 4.3 TB/s).
 // Three waves a SIMD, as many as its LDS allows, need 157 registers.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void gdn_chunk_operands_kernel(const GdnRecurArgs a,
                                                                  uint16_t* __restrict__ ws,

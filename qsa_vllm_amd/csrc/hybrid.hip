@@ -11,18 +11,21 @@
 //    n * bf16(sigmoid(bf16(up(bf16(silu(bf16(down(n)))))))) of YuLanGatedNorm,
 //    16 tokens per workgroup, the rank-16 projections on MFMA;
 //  * silu_mul_kernel: bf16(silu(g) * u) in fp32 (SiluAndMul);
-//  * gdn_prep_kernel: per token, the depthwise causal convolution of the
+//  * gdn_prep_kernel: the depthwise causal convolution of the
 //    projected q|k|v channels over the sequence's last K-1 inputs (from the
 //    conv state before the chunk) with SiLU, rounded to bf16; l2-normalised
 //    q (times dk^-1/2) and k in fp32; the gates g = -exp(A_log) *
 //    softplus(a + dt_bias) and beta = sigmoid(b);
 //  * gdn_conv_state_kernel: the new conv state (each sequence's last K-1
 //    inputs), after the prep kernel has read the old one;
-//  * gdn_recurrence_kernel: the gated delta rule per (sequence, value head)
-//    over the sequence's tokens in order, state S [dk, dv] fp32 held in
+//  * gdn_recurrence_kernel (gdn_device.h): the gated delta rule per (sequence,
+//    value head) over the sequence's tokens in order, state S [dk, dv] fp32 held in
 //    registers (lane (w, l) of the 4 waves owns column 32 w + (l & 31),
 //    rows 64 (l >> 5) .. + 63): S <- e^g S, u = beta (v - S^T k),
 //    S <- S + k u^T, o = S^T q;
+//  * gdn_chunk_kernel: the same rule in 64-token chunks, one launch, for
+//    batches of short prompts and callers without a workspace (gdn_scan.hip
+//    has the two-launch form);
 //  * gdn_norm_kernel: y = bf16(rmsnorm(o) * w * silu(z)) per (token, value head).
 //
 // Layouts: the GDN projection rows are grouped per key head as
