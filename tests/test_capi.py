@@ -92,6 +92,24 @@ def test_gated_norm_hidden_sizes_checked_before_the_row_split():
     assert lib.qsa_gated_norm(*(p + [0, 3072, 16, 1e-6, None, 0, None])) == 0   # no rows
 
 
+def test_gdn_recurrence_workspace_rule():
+    """Two-launch chunks: a slot per 64 tokens and one per sequence, 32 KiB per
+    key head and 19 KiB per value head each. None for batches known to hold no
+    sequence past one chunk, and none past 2 GiB (the one-launch kernel)."""
+    f = _lib.load().qsa_gdn_recurrence_workspace_bytes
+    slot = 8 * 32 * 1024 + 16 * 19 * 1024
+    assert f(8192, 1, 8, 16, 8192) == (128 + 1) * slot
+    assert f(8304, 128, 8, 16, 512) == (129 + 128) * slot
+    assert f(8304, 128, 8, 16, -1) == (129 + 128) * slot
+    assert f(65, 1, 8, 16, 65) == 2 * slot
+    for tokens, longest in ((64, -1), (8192, 64), (8192, 15), (8192, 0), (0, -1)):
+        assert f(tokens, 4, 8, 16, longest) == 0
+    most = (2 << 30) // slot - 1
+    assert f(64 * most, 1, 8, 16, -1) == (most + 1) * slot
+    assert f(64 * (most + 1), 1, 8, 16, -1) == 0
+    assert f(8192, 0, 8, 16, -1) == 0
+
+
 def test_workspace_and_split_helpers():
     lib = _lib.load()
     assert lib.qsa_sparse_attention_workspace_bytes(64, 16, 128, 1) == 0
