@@ -164,14 +164,18 @@ def gdn_recurrence(q, k, v, g, beta, state, query_start_loc, slots, key_heads, v
     o = torch.empty(tokens, value_heads, HEAD_DIM, dtype=torch.bfloat16, device=dev)
     num_seqs = query_start_loc.numel() - 1
     longest = -1 if max_query_len is None else int(max_query_len)
-    nbytes = _lib.load().qsa_gdn_recurrence_workspace_bytes(tokens, num_seqs, key_heads,
-                                                            value_heads, longest)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    args = (_ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta), tokens, _ptr(state), state.size(0),
+            _ptr(query_start_loc), _ptr(slots), num_seqs, key_heads, value_heads, HEAD_DIM,
+            longest, _ptr(o))
+    # No sequence past one chunk of 64 tokens (a decode batch): no workspace to ask for.
+    nbytes = 0 if 0 <= longest <= 64 else _lib.load().qsa_gdn_recurrence_workspace_bytes(
+        tokens, num_seqs, key_heads, value_heads, longest)
     with torch.cuda.device(dev):
-        _lib.call("qsa_gdn_recurrence_ws", _ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta), tokens,
-                  _ptr(state), state.size(0), _ptr(query_start_loc), _ptr(slots), num_seqs,
-                  key_heads, value_heads, HEAD_DIM, longest, _ptr(o), _ptr(ws), nbytes,
-                  _stream(dev))
+        if nbytes:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            _lib.call("qsa_gdn_recurrence_ws", *args, _ptr(ws), nbytes, _stream(dev))
+        else:
+            _lib.call("qsa_gdn_recurrence", *args, _stream(dev))
     return o
 
 
