@@ -2,12 +2,12 @@
 // (hybrid.hip, gdn_scan.hip).
 #pragma once
 
+#include "gdn_plan.h"
 #include "qsa_common.h"
 
 namespace qsa {
 
 constexpr int kHeadDim = 128;
-constexpr int kGdnChunkMin = 16;  // sequences this long take a chunked kernel
 
 struct GdnRecurArgs {
   const float* q;  // [tokens, key_heads, 128]

@@ -1,0 +1,64 @@
+// Host rules of the chunked gated delta rule (no HIP: the host tests compile this file alone).
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+namespace qsa {
+
+constexpr int kGdnChunk = 64;     // tokens per chunk
+constexpr int kGdnChunkMin = 16;  // sequences this long take a chunked kernel
+
+// Whether a batch runs the two-launch chunked form (gdn_scan.hip) instead of
+// gdn_chunk_kernel and gdn_recurrence_kernel. max_seq_tokens < 0: unknown.
+//
+// The one-launch kernel walks a (sequence, value head) pair's chunks in one
+// workgroup, ~16 us a chunk, 256 pairs (one a CU) side by side; the two
+// launches cost ~23 us and then ~1 us a chunk, with up to 128 pairs side by
+// side where there are many. So they win with the length of the longest
+// sequence. Times one-launch / two-launch, us, 16 value heads:
+//  * up to one chunk there is nothing to walk: 16 sequences of 60 tokens 25 / 40;
+//  * two chunks: two launches, unless the pairs end in the second half of the
+//    one-launch kernel's first or second round (129-256, 385-512 pairs): 8 x 66
+//    tokens 34 / 29, 9 x 66 35 / 39, 16 x 66 37 / 44, 16 x 128 41 / 49, 17 x 66
+//    66 / 53, 24 x 96 70 / 59, 25 x 66 69 / 77, 32 x 96 75 / 82, 33 x 96 103 / 87,
+//    48 x 96 109 / 107, 64 x 128 152 / 143. Single chunks beside a sequence of
+//    two gain nothing: 24 x 33 and one of 66 42 / 52, 60 x 64 and one of 66 88 / 121;
+//  * three chunks and more: 16 x 130 52 / 52, 16 x 256 71 / 58, 16 x 400 111 / 90,
+//    one of 8192 1812 / 161;
+//  * decode sequences run in the first of the two launches, but each puts empty
+//    workgroups into the walk: 120 and one prompt of 100 77 / 61, 250 117 / 117,
+//    500 223 / 228; of 200: 500 251 / 243, 1000 436 / 448; of 500: 1000 496 / 481.
+//    32 and more of them hide what a half-empty round of two-chunk sequences
+//    loses: 32 and 16 x 66 50 / 51, 112 and 16 x 66 83 / 73;
+//  * unknown lengths: 100 decode requests 43 / 48, 200 x 3 tokens 91 / 95.
+// Where many sequences of 16 to 64 tokens accompany a much longer one, the
+// sizes known here do not tell them from decode requests beside several
+// prompts: 128 x 64 and one of 512 190 / 260, but 112 decode requests and 16 x
+// 512, of the same token count, 172 / 139. They are taken for the latter.
+inline bool gdn_two_launches(int tokens, int num_seqs, int value_heads, int max_seq_tokens) {
+  if (tokens <= kGdnChunk || num_seqs <= 0) return false;
+  if (max_seq_tokens < 0) return tokens / 4 >= num_seqs;
+  const int64_t longest = std::min(max_seq_tokens, tokens);
+  if (longest <= kGdnChunk) return false;
+  const int64_t chunks = (longest + kGdnChunk - 1) / kGdnChunk, n = num_seqs;
+  const auto rounds_pay = [](int64_t pairs) {
+    const int64_t halves = (pairs + 127) / 128;
+    return halves != 2 && halves != 4;
+  };
+  const int64_t others = n > 1 ? (tokens - longest) / (n - 1) : 0;  // their mean length
+  if (n > 1 && others < 32) {
+    // Decode sequences among them: the tokens past one per sequence are taken
+    // to be in sequences as long as the longest.
+    const int64_t extra = std::max<int64_t>(tokens - n, 1);
+    const int64_t longs = std::min(n, (extra + longest - 2) / (longest - 1));
+    const int64_t short_pairs = (n - longs) * value_heads;
+    if (short_pairs >= 5600 * chunks - 7700) return false;
+    return chunks > 2 || short_pairs >= 512 || rounds_pay(longs * value_heads);
+  }
+  if (chunks > 2) return true;
+  const int64_t pairs = n * value_heads;
+  return pairs <= 128 || (others > kGdnChunk && rounds_pay(pairs));
+}
+
+}  // namespace qsa

@@ -25,7 +25,7 @@ namespace qsa {
 namespace {
 
 constexpr int kDim = 128;
-constexpr int kC = 64;  // tokens per chunk
+constexpr int kC = kGdnChunk;  // tokens per chunk
 // A fragment is one MFMA operand of a wave: 64 lanes x 8 bf16.
 constexpr int kFrag = 512;  // bf16 elements
 // Per (chunk, key head): K and Q, 16 fragments each.

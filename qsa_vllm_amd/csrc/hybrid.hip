@@ -25,7 +25,7 @@
 //    S <- S + k u^T, o = S^T q;
 //  * gdn_chunk_kernel: the same rule in 64-token chunks, one launch, for
 //    batches of short prompts and callers without a workspace (gdn_scan.hip
-//    has the two-launch form);
+//    has the two-launch form, gdn_plan.h the rule between them);
 //  * gdn_norm_kernel: y = bf16(rmsnorm(o) * w * silu(z)) per (token, value head).
 //
 // Layouts: the GDN projection rows are grouped per key head as
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(256) void gdn_recurrence_kernel(const GdnRecurArgs 
 // solve are fp32: 16-row blocks, each taking the earlier blocks' contribution
 // and the inverse of its diagonal block as fp32 MFMA work.
 // ---------------------------------------------------------------------------
-constexpr int kChunk = 64;
+constexpr int kChunk = kGdnChunk;
 
 struct ChunkLds {
   uint16_t q[kChunk][136];        // bf16 q (normalised, scaled)
@@ -1223,11 +1223,8 @@ int gdn_recurrence(const float* q, const float* k, const void* v, const float* g
 
 extern "C" size_t qsa_gdn_recurrence_workspace_bytes(int tokens, int num_seqs, int key_heads,
                                                      int value_heads, int max_seq_tokens) {
-  // Sequences of a single chunk stay on the one-launch kernel: there is nothing
-  // to walk, and it saves the operands' round trip through memory (16 of 60
-  // tokens 25 us against 40, 64 of 60 tokens 91 against 94).
-  if (tokens <= 0 || num_seqs <= 0 || key_heads <= 0 || value_heads <= 0 || tokens <= kChunk ||
-      (max_seq_tokens >= 0 && max_seq_tokens <= kChunk) ||
+  if (tokens <= 0 || num_seqs <= 0 || key_heads <= 0 || value_heads <= 0 ||
+      !gdn_two_launches(tokens, num_seqs, value_heads, max_seq_tokens) ||
       (int64_t)num_seqs * value_heads > 0x7fffffffLL / 8 || (int64_t)num_seqs + tokens > 0x7fffffffLL)
     return 0;
   const size_t bytes = gdn_scan_workspace_bytes(tokens, num_seqs, key_heads, value_heads);

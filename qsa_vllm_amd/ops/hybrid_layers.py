@@ -167,8 +167,8 @@ def gdn_recurrence(q, k, v, g, beta, state, query_start_loc, slots, key_heads, v
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta), tokens, _ptr(state), state.size(0),
             _ptr(query_start_loc), _ptr(slots), num_seqs, key_heads, value_heads, HEAD_DIM,
             longest, _ptr(o))
-    # No sequence past one chunk of 64 tokens (a decode batch): no workspace to ask for.
-    nbytes = 0 if 0 <= longest <= 64 else _lib.load().qsa_gdn_recurrence_workspace_bytes(
+    # A decode batch asks for no workspace, without a call to find out.
+    nbytes = 0 if 0 <= longest <= 1 else _lib.load().qsa_gdn_recurrence_workspace_bytes(
         tokens, num_seqs, key_heads, value_heads, longest)
     with torch.cuda.device(dev):
         if nbytes:

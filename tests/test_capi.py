@@ -110,6 +110,42 @@ def test_gdn_recurrence_workspace_rule():
     assert f(8192, 0, 8, 16, -1) == 0
 
 
+def test_gdn_recurrence_form_rule():
+    """Which batches of the delta rule run the two-launch chunks (a workspace is
+    asked for): those measured to be no slower that way. Batches (sequence
+    lengths, longest known or not, two launches) at 16 value heads."""
+    f = _lib.load().qsa_gdn_recurrence_workspace_bytes
+
+    def two(lens, known=True, heads=(8, 16)):
+        return f(sum(lens), len(lens), *heads, max(lens) if known else -1) > 0
+
+    for n, m in ((1, 65), (8, 66), (8, 128), (17, 66), (24, 96), (33, 100), (64, 128), (16, 130),
+                 (16, 256), (64, 192), (1, 8192), (3, 2700)):
+        assert two([m] * n), (n, m)
+    for n, m in ((9, 66), (10, 128), (12, 100), (16, 66), (16, 128), (25, 66), (32, 66), (32, 128)):
+        assert not two([m] * n), (n, m)
+    assert two([66] * 16, heads=(4, 8)) and not two([66] * 32, heads=(4, 8))
+    assert two([128] * 4, heads=(16, 32)) and not two([66] * 8, heads=(16, 32))
+    # Single-chunk sequences with one of two chunks; few of them are no loss.
+    assert not two([64] * 60 + [66]) and not two([40] * 100 + [65]) and not two([16] * 400 + [80])
+    assert not two([33] * 24 + [66]) and two([33] * 7 + [128]) and two([40, 128])
+    # Decode sequences beside prompts.
+    for nd, m in ((8, 66), (120, 100), (120, 65), (200, 65), (500, 200), (500, 500), (900, 2000)):
+        assert two([1] * nd + [m]), (nd, m)
+    for nd, m in ((500, 65), (500, 100), (1000, 65), (1000, 200)):
+        assert not two([1] * nd + [m]), (nd, m)
+    assert two([1] * 112 + [512] * 16) and two([1] * 112 + [66] * 16) and two([1] * 32 + [100] * 8)
+    # Unknown lengths: a decode batch, drafted tokens; prompts.
+    for lens in ([1] * 65, [1] * 1000, [3] * 200, [64]):
+        assert not two(lens, known=False), lens[:2]
+    for lens in ([8192], [512] * 16, [1] * 100 + [8000]):
+        assert two(lens, known=False), lens[:2]
+    # A bound past the batch is the batch; sequences without tokens.
+    assert f(8192, 1, 8, 16, 2 ** 31 - 1) == f(8192, 1, 8, 16, 8192) > 0
+    assert f(65, 300, 8, 16, 65) == 0 and f(65, 3, 8, 16, 65) > 0
+    assert f(2 ** 31 - 1, 1, 8, 16, 2 ** 31 - 1) == 0    # past 2 GiB
+
+
 def test_workspace_and_split_helpers():
     lib = _lib.load()
     assert lib.qsa_sparse_attention_workspace_bytes(64, 16, 128, 1) == 0
