@@ -61,4 +61,18 @@ inline bool gdn_two_launches(int tokens, int num_seqs, int value_heads, int max_
   return pairs <= 128 || (others > kGdnChunk && rounds_pay(pairs));
 }
 
+// Workspace slots of the two-launch form, one per chunk: sequence `seq`'s chunks
+// take consecutive ones from gdn_first_slot on. Between two sequences of
+// kGdnChunkMin tokens or more seq and start / 16 both grow, so their minimum
+// does; with floor(start / 64) + ceil(len / 64) - 1 <= floor((start + len) / 64),
+// no two chunks share a slot and all are below gdn_slots. A slot per sequence
+// beside those per 64 tokens would serve too, but 900 decode requests beside a
+// prompt of 2000 tokens need 226 this way and 946 that way.
+constexpr int gdn_first_slot(int start, int seq) {
+  return start / kGdnChunk + (seq < start / kGdnChunkMin ? seq : start / kGdnChunkMin);
+}
+constexpr int64_t gdn_slots(int tokens, int num_seqs) {
+  return (int64_t)tokens / kGdnChunk + (num_seqs < tokens / kGdnChunkMin ? num_seqs : tokens / kGdnChunkMin);
+}
+
 }  // namespace qsa

@@ -57,9 +57,7 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Sequence i's chunks take the workspace slots start / 64 + i onwards:
-// floor(start / 64) + ceil(len / 64) - 1 <= floor((start + len) / 64), so
-// consecutive sequences never share one and all are below tokens / 64 + num_seqs.
+// The sequences that take the chunked kernels (gdn_first_slot has their workspace slots).
 __device__ __forceinline__ bool chunked_sequence(const GdnRecurArgs& a, int seq, int* start, int* len) {
   *start = a.seq_start[seq];
   *len = a.seq_start[seq + 1] - *start;
@@ -105,7 +103,7 @@ __device__ __forceinline__ void chunk_operands(const GdnRecurArgs& a, uint16_t* 
     const int i = min(i0 + lane, a.num_seqs - 1);
     int s0, n;
     const bool chunked = chunked_sequence(a, i, &s0, &n);
-    const int at = slot - (s0 / kC + i);
+    const int at = slot - gdn_first_slot(s0, i);
     const uint64_t hit = __ballot(chunked && at >= 0 && at < (n + kC - 1) / kC);
     if (hit) {
       const int src = __builtin_ctzll(hit);
@@ -115,7 +113,7 @@ __device__ __forceinline__ void chunk_operands(const GdnRecurArgs& a, uint16_t* 
     }
   }
   if (seq < 0) return;
-  const int c0 = (slot - (start / kC + seq)) * kC;
+  const int c0 = (slot - gdn_first_slot(start, seq)) * kC;
   const int nc = min(kC, len - c0);
   const int r = a.value_heads / a.key_heads;
 
@@ -411,7 +409,7 @@ __global__ __launch_bounds__(64 * (SW + 2)) __attribute__((amdgpu_waves_per_eu(2
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g = lane >> 4;
   const int chunks = (len + kC - 1) / kC;
-  const int64_t slot0 = start / kC + seq;
+  const int64_t slot0 = gdn_first_slot(start, seq);
   const int hk = h / (a.value_heads / a.key_heads);
   const int64_t key_stride = (int64_t)a.key_heads * kKeyElems;
   const int64_t val_stride = (int64_t)a.value_heads * kValElems;
@@ -681,8 +679,6 @@ __global__ __launch_bounds__(64 * (SW + 2)) __attribute__((amdgpu_waves_per_eu(2
   }
 }
 
-int64_t workspace_slots(int tokens, int num_seqs) { return (int64_t)tokens / kC + num_seqs; }
-
 template <int NL, int SW, int BUF>
 void launch_scan(const GdnRecurArgs& a, const uint16_t* ws, int slots, hipStream_t stream) {
   const unsigned parts = kDim / ScanLds<NL, SW, BUF>::kCols;
@@ -693,12 +689,12 @@ void launch_scan(const GdnRecurArgs& a, const uint16_t* ws, int slots, hipStream
 }  // namespace
 
 size_t gdn_scan_workspace_bytes(int tokens, int num_seqs, int key_heads, int value_heads) {
-  return (size_t)workspace_slots(tokens, num_seqs) * 2 *
+  return (size_t)gdn_slots(tokens, num_seqs) * 2 *
          ((size_t)key_heads * kKeyElems + (size_t)value_heads * kValElems);
 }
 
 int gdn_scan_launch(const GdnRecurArgs& a, int max_seq_tokens, void* workspace, hipStream_t stream) {
-  const int slots = (int)workspace_slots(a.tokens, a.num_seqs);
+  const int slots = (int)gdn_slots(a.tokens, a.num_seqs);
   uint16_t* ws = static_cast<uint16_t*>(workspace);
   hipLaunchKernelGGL(gdn_chunk_operands_kernel, 
                      dim3((unsigned)(slots * a.key_heads + a.num_seqs * a.value_heads)), dim3(256), 0, stream, a, ws, slots);

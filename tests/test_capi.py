@@ -146,6 +146,57 @@ def test_gdn_recurrence_form_rule():
     assert f(2 ** 31 - 1, 1, 8, 16, 2 ** 31 - 1) == 0    # past 2 GiB
 
 
+def test_gdn_recurrence_workspace_counts_chunkable_sequences():
+    """Sequences below 16 tokens take no workspace slot: at most tokens / 16 do."""
+    f = _lib.load().qsa_gdn_recurrence_workspace_bytes
+    slot = 8 * 32 * 1024 + 16 * 19 * 1024
+    assert f(2900, 901, 8, 16, 2000) == (2900 // 64 + 2900 // 16) * slot
+    assert f(2112, 113, 8, 16, 2000) == (2112 // 64 + 113) * slot
+    assert f(100, 5, 8, 16, 96) == (1 + 5) * slot
+    assert f(79, 5, 8, 16, 75) == (1 + 4) * slot
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_gdn_workspace_slots_host(tmp_path):
+    """Every chunk of random batches (sequences of 0-15 tokens between longer
+    ones) has a slot of its own, below the count that the workspace holds."""
+    src = tmp_path / "slots.cpp"
+    src.write_text(r'''
+#include "gdn_plan.h"
+#include <cstdio>
+#include <random>
+#include <vector>
+int main() {
+  std::mt19937 rng(7);
+  for (int trial = 0; trial < 20000; ++trial) {
+    const int n = 1 + rng() % (trial % 5 ? 12 : 300), shape = rng() % 4;
+    std::vector<int> start{0};
+    for (int i = 0; i < n; ++i) {
+      const int len = shape == 0 ? rng() % 16 : shape == 1 ? 16 + rng() % 3 : rng() % 5 ? rng() % 17 : rng() % 400;
+      start.push_back(start.back() + len);
+    }
+    const int64_t slots = qsa::gdn_slots(start[n], n);
+    std::vector<char> used(slots, 0);
+    for (int i = 0; i < n; ++i) {
+      const int len = start[i + 1] - start[i];
+      for (int c = 0; len >= qsa::kGdnChunkMin && c * qsa::kGdnChunk < len; ++c) {
+        const int at = qsa::gdn_first_slot(start[i], i) + c;
+        if (at < 0 || at >= slots || used[at]) { printf("FAIL %d %d\\n", trial, i); return 1; }
+        used[at] = 1;
+      }
+    }
+  }
+  printf("OK\\n");
+  return 0;
+}
+''')
+    exe = tmp_path / "slots"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", str(ROOT / "qsa_vllm_amd" / "csrc"),
+                    str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and "OK" in out.stdout, out.stdout
+
+
 def test_workspace_and_split_helpers():
     lib = _lib.load()
     assert lib.qsa_sparse_attention_workspace_bytes(64, 16, 128, 1) == 0

@@ -586,6 +586,36 @@ def test_gdn_recurrence_chunk_edges(hk, hv, lens, bound):
         assert torch.equal(state[slot].cpu(), state0[slot])
 
 
+@pytest.mark.parametrize("num_seqs,chunked", [
+    (64, {0: 100, 63: 70}), (65, {0: 16, 63: 66, 64: 130}), (131, {0: 65, 63: 17, 64: 200, 130: 129})])
+def test_gdn_recurrence_chunks_among_many_sequences(num_seqs, chunked):
+    """The chunk operands find each workspace slot's sequence among more than 64,
+    one-token sequences between the chunked ones. Keys and limits as for the chunk edges."""
+    lens = [chunked.get(i, 1) for i in range(num_seqs)]
+    hk, hv, tokens = 1, 2, sum(lens)
+    gen = torch.Generator().manual_seed(num_seqs)
+    q = torch.nn.functional.normalize(torch.randn(tokens, hk, 128, generator=gen), dim=-1) / 128 ** 0.5
+    k = torch.nn.functional.normalize(torch.randn(tokens, hk, 128, generator=gen), dim=-1)
+    v = torch.randn(tokens, hv, 128, generator=gen).to(torch.bfloat16)
+    g = -0.01 * torch.rand(tokens, hv, generator=gen)
+    beta = torch.rand(tokens, hv, generator=gen)
+    state0 = 0.05 * torch.randn(num_seqs, hv, 128, 128, generator=gen)
+    starts = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32)
+    slots = torch.randperm(num_seqs, generator=gen)
+    state = state0.to(DEV)
+    print(f"[hybrid] gdn recurrence, {num_seqs} sequences, chunked {chunked}", flush=True)
+    assert L._lib.load().qsa_gdn_recurrence_workspace_bytes(tokens, num_seqs, hk, hv, max(lens)) > 0
+    o = L.gdn_recurrence(q.to(DEV), k.to(DEV), v.to(DEV), g.to(DEV), beta.to(DEV), state,
+                         starts.to(DEV), slots.to(DEV), hk, hv, max_query_len=max(lens))
+    torch.cuda.synchronize()
+    for i, m in enumerate(lens):
+        rows, slot = slice(int(starts[i]), int(starts[i]) + m), int(slots[i])
+        want_o, want_s = H.gated_delta_rule(q[rows].expand(-1, hv, -1), k[rows].expand(-1, hv, -1),
+                                            v[rows].float(), g[rows], beta[rows], state0[slot])
+        _close(o[rows].cpu(), want_o, f"output, sequence {i} of {m}")
+        _close(state[slot].cpu(), want_s, f"state, sequence {i} of {m}", 1e-2, 1e-3)
+
+
 @pytest.mark.parametrize("K,hk,hv,lens,shift", [
     (4, 2, 4, [1, 1, 2, 3, 1, 5, 4], 0),                       # one token per workgroup
     (4, 2, 4, [3, 1000, 1, 2, 1042], 0),                       # four
