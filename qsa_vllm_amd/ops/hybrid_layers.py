@@ -142,7 +142,9 @@ def gdn_recurrence(q, k, v, g, beta, state, query_start_loc, slots, key_heads, v
     """The gated delta rule over each sequence (state updated in place).
     Returns o [T, Hv, 128] bf16. ``max_query_len``: the longest sequence's
     token count when the caller knows it (a decode batch: 1); below 16 the
-    chunked kernel is not launched."""
+    chunked kernel is not launched. Batches that run the two-launch chunks take
+    a workspace for the call (``qsa_gdn_recurrence_workspace_bytes``, at most
+    2 GiB); if it cannot be allocated they run without it, slower."""
     dev = _on_gpu(q, k, v, g, beta, state, query_start_loc, slots)
     tokens = q.size(0)
     for t, name in ((q, "q"), (k, "k")):
@@ -171,8 +173,13 @@ def gdn_recurrence(q, k, v, g, beta, state, query_start_loc, slots, key_heads, v
     nbytes = 0 if 0 <= longest <= 1 else _lib.load().qsa_gdn_recurrence_workspace_bytes(
         tokens, num_seqs, key_heads, value_heads, longest)
     with torch.cuda.device(dev):
+        ws = None
         if nbytes:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            try:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            except torch.cuda.OutOfMemoryError:
+                pass  # a full card: the kernels that need none
+        if ws is not None:
             _lib.call("qsa_gdn_recurrence_ws", *args, _ptr(ws), nbytes, _stream(dev))
         else:
             _lib.call("qsa_gdn_recurrence", *args, _stream(dev))

@@ -586,6 +586,42 @@ def test_gdn_recurrence_chunk_edges(hk, hv, lens, bound):
         assert torch.equal(state[slot].cpu(), state0[slot])
 
 
+def test_gdn_recurrence_without_memory_for_its_workspace(monkeypatch):
+    """A card too full for the workspace: the call runs the kernels that need none."""
+    gen = torch.Generator().manual_seed(61)
+    hk, hv, lens = 1, 2, [150, 1, 40]
+    tokens = sum(lens)
+    unit = lambda: torch.nn.functional.normalize(torch.randn(tokens, hk, 128, generator=gen), dim=-1)  # noqa: E731
+    q, k = unit() / 128 ** 0.5, unit()
+    v = torch.randn(tokens, hv, 128, generator=gen).to(torch.bfloat16)
+    g, beta = -0.1 * torch.rand(tokens, hv, generator=gen), torch.rand(tokens, hv, generator=gen)
+    state0 = 0.05 * torch.randn(3, hv, 128, 128, generator=gen)
+    starts = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32)
+    args = [t.to(DEV) for t in (q, k, v, g, beta)]
+    state = state0.to(DEV)
+    empty, asked = torch.empty, []
+
+    def full(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            asked.append(size)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    starts_dev, slots = starts.to(DEV), torch.arange(3, device=DEV)
+    monkeypatch.setattr(torch, "empty", full)
+    print("[hybrid] gdn recurrence, workspace refused", flush=True)
+    o = L.gdn_recurrence(*args, state, starts_dev, slots, hk, hv, max_query_len=150)
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    assert asked
+    for i, m in enumerate(lens):
+        rows = slice(int(starts[i]), int(starts[i]) + m)
+        want_o, want_s = H.gated_delta_rule(q[rows].expand(-1, hv, -1), k[rows].expand(-1, hv, -1),
+                                            v[rows].float(), g[rows], beta[rows], state0[i])
+        _close(o[rows].cpu(), want_o, f"output, sequence of {m}")
+        _close(state[i].cpu(), want_s, f"state, sequence of {m}", 1e-2, 1e-3)
+
+
 @pytest.mark.parametrize("num_seqs,chunked", [
     (64, {0: 100, 63: 70}), (65, {0: 16, 63: 66, 64: 130}), (131, {0: 65, 63: 17, 64: 200, 130: 129})])
 def test_gdn_recurrence_chunks_among_many_sequences(num_seqs, chunked):
