@@ -463,9 +463,13 @@ int qsa_gdn_recurrence(const float* q, const float* k, const void* v, const floa
                        void* stream);
 
 /* The same with a workspace for the two-launch chunked kernels, which spread a
- * long sequence over many compute units. Bytes needed (0: the call uses none,
- * as for a decode batch). A null workspace, or an o that is not 16-byte aligned,
- * runs qsa_gdn_recurrence's kernels. */
+ * long sequence over many compute units. qsa_gdn_recurrence_workspace_bytes: the
+ * bytes needed, at most 2 GiB (0: the call uses none, as for a decode batch). A
+ * null workspace, or an o that is not 16-byte aligned, runs qsa_gdn_recurrence's
+ * kernels. A workspace that is too small or not 16-byte aligned is
+ * QSA_ERR_WORKSPACE, and nothing runs. It holds the call's data until the call's
+ * work is done: calls that may overlap (other streams, other threads) need one
+ * each. */
 size_t qsa_gdn_recurrence_workspace_bytes(int tokens, int num_seqs, int key_heads, int value_heads,
                                           int max_seq_tokens);
 int qsa_gdn_recurrence_ws(const float* q, const float* k, const void* v, const float* g,

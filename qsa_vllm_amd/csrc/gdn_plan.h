@@ -75,4 +75,18 @@ constexpr int64_t gdn_slots(int tokens, int num_seqs) {
   return (int64_t)tokens / kGdnChunk + (num_seqs < tokens / kGdnChunkMin ? num_seqs : tokens / kGdnChunkMin);
 }
 
+// Value columns per workgroup of the walk: the narrowest slices whose workgroups
+// fit the chip's 256 CUs at once (LDS holds one workgroup a CU). A workgroup's
+// time per chunk hardly depends on its width, so more of them only help while
+// they run side by side. Long sequences of the batch: at least tokens /
+// max_seq_tokens. Measured, both launches, 16 value heads, 8192 tokens (16 / 32 /
+// 64 columns, us): one sequence 164 / 173 / 248, two 114 / 113 / 152, four
+// 114 / 85 / 103, eight 128 / 95 / 84, sixteen 204 / 129 / 97.
+inline int gdn_scan_columns(int tokens, int num_seqs, int value_heads, int max_seq_tokens) {
+  const int64_t longest = std::min(max_seq_tokens, tokens);  // a bound may be any int
+  const int64_t side = max_seq_tokens > 0 ? (tokens + longest - 1) / longest : num_seqs;
+  const int64_t pairs = side * value_heads;
+  return pairs * 8 <= 256 ? 16 : pairs * 4 <= 256 ? 32 : 64;
+}
+
 }  // namespace qsa

@@ -700,18 +700,11 @@ int gdn_scan_launch(const GdnRecurArgs& a, int max_seq_tokens, void* workspace, 
                      dim3((unsigned)(slots * a.key_heads + a.num_seqs * a.value_heads)), dim3(256), 0, stream, a, ws, slots);
   const int st = check_launch("qsa_gdn_recurrence (chunk operands)");
   if (st != QSA_OK) return st;
-  // The narrowest slices whose workgroups fit the chip's 256 CUs at once (LDS
-  // holds one workgroup a CU): a workgroup's time per chunk hardly depends on
-  // its width, so more of them only help while they run side by side. Long
-  // sequences of the batch: at least tokens / max_seq_tokens. Measured, both
-  // launches, 16 value heads, 8192 tokens (<1, 1> / <1, 2> / <2, 2>, us): one
-  // sequence 164 / 173 / 248, two 114 / 113 / 152, four 114 / 85 / 103, eight
-  // 128 / 95 / 84, sixteen 204 / 129 / 97.
-  const int64_t side = max_seq_tokens > 0 ? (a.tokens + max_seq_tokens - 1) / max_seq_tokens : a.num_seqs;
-  const int64_t pairs = side * a.value_heads;
-  if (pairs * 8 <= 256) launch_scan<1, 1, 3>(a, ws, slots, stream);
-  else if (pairs * 4 <= 256) launch_scan<1, 2, 2>(a, ws, slots, stream);
-  else launch_scan<2, 2, 2>(a, ws, slots, stream);
+  switch (gdn_scan_columns(a.tokens, a.num_seqs, a.value_heads, max_seq_tokens)) {
+    case 16: launch_scan<1, 1, 3>(a, ws, slots, stream); break;
+    case 32: launch_scan<1, 2, 2>(a, ws, slots, stream); break;
+    default: launch_scan<2, 2, 2>(a, ws, slots, stream); break;
+  }
   return check_launch("qsa_gdn_recurrence (scan)");
 }
 

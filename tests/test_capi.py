@@ -197,6 +197,41 @@ int main() {
     assert out.returncode == 0 and "OK" in out.stdout, out.stdout
 
 
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_gdn_scan_columns_host(tmp_path):
+    """Slice widths of the walk: narrow while the workgroups fit the chip; any
+    bound past the batch's tokens is the batch's tokens."""
+    src = tmp_path / "columns.cpp"
+    src.write_text(r'''
+#include "gdn_plan.h"
+#include <cstdio>
+#include <initializer_list>
+int main() {
+  struct { int tokens, seqs, heads, longest, columns; } cases[] = {
+      {8192, 1, 16, 8192, 16}, {8192, 2, 16, 4096, 16}, {8192, 4, 16, 2048, 32}, {8192, 8, 16, 1024, 64},
+      {8304, 128, 16, 512, 64}, {8192, 4, 16, -1, 32}, {8192, 1, 32, 8192, 16}, {65, 2, 64, 64, 64}};
+  for (auto& c : cases)
+    if (qsa::gdn_scan_columns(c.tokens, c.seqs, c.heads, c.longest) != c.columns) {
+      printf("FAIL %d %d %d\\n", c.tokens, c.heads, c.longest);
+      return 1;
+    }
+  for (int heads : {1, 16, 64, 128})
+    for (int longest : {8192, 8193, 2147483647 - 8192, 2147483647 - 8191, 2147483647})
+      if (qsa::gdn_scan_columns(8192, 3, heads, longest) != qsa::gdn_scan_columns(8192, 3, heads, 8192)) {
+        printf("FAIL bound %d\\n", longest);
+        return 1;
+      }
+  printf("OK\\n");
+  return 0;
+}
+''')
+    exe = tmp_path / "columns"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", str(ROOT / "qsa_vllm_amd" / "csrc"),
+                    str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and "OK" in out.stdout, out.stdout
+
+
 def test_workspace_and_split_helpers():
     lib = _lib.load()
     assert lib.qsa_sparse_attention_workspace_bytes(64, 16, 128, 1) == 0
