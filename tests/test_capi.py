@@ -146,6 +146,22 @@ def test_gdn_recurrence_form_rule():
     assert f(2 ** 31 - 1, 1, 8, 16, 2 ** 31 - 1) == 0    # past 2 GiB
 
 
+def test_gdn_recurrence_workspace_errors_need_no_launch():
+    """A workspace that is short or misaligned is refused before any launch."""
+    lib = _lib.load()
+    need = lib.qsa_gdn_recurrence_workspace_bytes(300, 2, 8, 16, 200)
+
+    def call(workspace, nbytes, o=1 << 26, tokens=300):
+        return lib.qsa_gdn_recurrence_ws(1 << 20, 1 << 21, 1 << 22, 1 << 23, 1 << 24, tokens, 1 << 25, 4,
+                                         1 << 27, 1 << 28, 2, 8, 16, 128, 200, o, workspace, nbytes, None)
+
+    for workspace, nbytes in ((1 << 30, need - 1), (1 << 30, 0), ((1 << 30) + 8, need), ((1 << 30) + 2, 2 * need)):
+        assert call(workspace, nbytes) == -4, (workspace, nbytes)
+        assert b"workspace" in lib.qsa_last_error()
+    assert call(1 << 30, 0, tokens=0) == 0
+    assert call(1 << 30, need, o=None) == -1
+
+
 def test_gdn_recurrence_workspace_counts_chunkable_sequences():
     """Sequences below 16 tokens take no workspace slot: at most tokens / 16 do."""
     f = _lib.load().qsa_gdn_recurrence_workspace_bytes
