@@ -367,6 +367,30 @@ def test_torch_ops_meta_kernels_trace_shapes():
         None, None, True, 0)
 
 
+def test_decode_layer_traces_and_refuses_host_tensors():
+    """The one-op decode step on meta tensors (shape-only tracing writes nothing,
+    returns nothing), its mutated arguments, and host tensors."""
+    import torch
+
+    import qsa_vllm_amd.ops  # noqa: F401
+
+    op = torch.ops.yulan_qsa_kernels.decode_layer
+    schema = op.default._schema
+    assert [a.name for a in schema.arguments if a.alias_info] == ["indices", "counts", "out"]
+
+    def call(device, gate):
+        e = lambda *s, dtype=torch.bfloat16: torch.empty(s, dtype=dtype, device=device)  # noqa: E731
+        i32 = torch.int32
+        return op(e(6, 32, 128), e(8, 16, 1, 128), e(4, 2, dtype=i32), e(6, dtype=i32), e(6, 16, 128),
+                  e(64, 16, 2, 128), e(64, 16, 2, 128), e(4, 32, dtype=i32), e(6, dtype=i32),
+                  e(6, dtype=torch.int64), e(4, dtype=i32), 4, 1024, 16, e(6, 2063, dtype=i32),
+                  e(6, dtype=i32), e(6, 16, 128), e(6, 16, 128) if gate else None)
+
+    assert call("meta", False) is None and call("meta", True) is None
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        call("cpu", False)
+
+
 def test_decode_select_attention_fusion_rule():
     """Which decode batch shapes the combined selection + attention runs as one
     launch: the top-k's 512-thread shapes (fewer than 1024 rows, at most 2048

@@ -239,3 +239,64 @@ def test_decode_select_attend_graph_replays():
         torch.cuda.synchronize()
         assert torch.equal(idx, want[0]) and torch.equal(counts, want[1]), rep
         assert torch.equal(out.view(torch.int16), want[2].view(torch.int16)), rep
+
+
+def _layer_tensors(wl, extra):
+    """Per-row tensors of a batch with ``extra`` padding rows, and its outputs, filled."""
+    s = wl.shape
+    pad = lambda t: torch.cat([t, t[:1].expand(extra, *t.shape[1:])]) if t is not None else None  # noqa: E731
+    rows = wl.rows + extra
+    return dict(index_q=pad(wl.q_index), visible=pad(wl.visible), q=pad(wl.q), t2r=pad(wl.token_to_req),
+                pos=pad(wl.positions), gate=pad(wl.gate),
+                idx=torch.full((rows, s.width), -9, dtype=torch.int32, device=wl.device),
+                counts=torch.full((rows,), -9, dtype=torch.int32, device=wl.device),
+                out=torch.full((rows, *wl.q.shape[1:]), 3.0, dtype=wl.q.dtype, device=wl.device))
+
+
+def _decode_layer(wl, t, count, columns):
+    torch.ops.yulan_qsa_kernels.decode_layer(
+        t["index_q"], wl.index_cache, wl.index_table, t["visible"], t["q"], wl.k_cache, wl.v_cache,
+        wl.block_table, t["t2r"], t["pos"], wl.seq_lens, count, columns, wl.shape.compress_ratio,
+        t["idx"], t["counts"], t["out"], t["gate"])
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("extra", [0, 3])
+@pytest.mark.parametrize("overrides", [{"batch": 5, "seed": 41}, {"batch": 8, "gate": True, "seed": 42},
+                                       {"batch": 6, "kv_layout": "head_major", "seed": 43}])
+def test_decode_layer_op(overrides, extra):
+    """One op on the first rows of whole-batch tensors: the selection, counts and
+    output of the calls it stands for on those rows, zeros past them in the
+    output, nothing past them in the buffers; no rows: zeros only."""
+    wl = make_workload("decode_32k", device="cuda:0", **overrides)
+    print(f"[decode layer] {overrides} extra {extra}", flush=True)
+    logits = _logits(wl)
+    idx, counts, out = _two_calls(wl, logits, 0, False)
+    t = _layer_tensors(wl, extra)
+    _decode_layer(wl, t, wl.rows, logits.shape[1])
+    n = wl.rows
+    assert torch.equal(t["idx"][:n], idx) and torch.equal(t["counts"][:n], counts)
+    assert torch.equal(t["out"][:n].view(torch.int16), out.view(torch.int16))
+    assert (t["out"][n:] == 0).all() and (t["idx"][n:] == -9).all() and (t["counts"][n:] == -9).all()
+    t = _layer_tensors(wl, extra)
+    _decode_layer(wl, t, 0, logits.shape[1])
+    assert (t["out"] == 0).all() and (t["idx"] == -9).all() and (t["counts"] == -9).all()
+
+
+def test_decode_layer_refusals():
+    wl = make_workload("decode_32k", device="cuda:0", batch=4, gate=True, seed=44)
+    columns = _logits(wl).shape[1]
+    print("[decode layer] refusals", flush=True)
+    for change, count, cols in (
+            ({}, -1, columns), ({}, 4, 0),
+            ({"idx": lambda x: x[:3]}, 4, columns), ({"idx": lambda x: x.long()}, 4, columns),
+            ({"counts": lambda x: x[:3]}, 4, columns), ({"out": lambda x: x[:3]}, 4, columns),
+            ({"out": lambda x: x.float()}, 4, columns), ({"gate": lambda x: x[:, :1]}, 4, columns),
+            ({"t2r": lambda x: x[:2]}, 4, columns), ({"pos": lambda x: x.int()}, 4, columns),
+            ({"visible": lambda x: x[:3]}, 4, columns), ({"q": lambda x: x[:3]}, 4, columns),
+            ({"index_q": lambda x: x.float()}, 4, columns), ({"q": lambda x: x.cpu()}, 4, columns)):
+        t = _layer_tensors(wl, 0)
+        for name, f in change.items():
+            t[name] = f(t[name])
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            _decode_layer(wl, t, count, cols)
