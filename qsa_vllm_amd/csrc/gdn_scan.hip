@@ -18,6 +18,16 @@
 // 8192 tokens kept 16 workgroups busy for 1812 us. Here it takes 44 us for the
 // operands (73 MB written, 67 MB of fp32 q and k read) and 117 us for the walk
 // (0.9 us a chunk, bound by the state waves' chain of products).
+//
+// Bits: gdn_chunk_kernel solves for U in fp32. Here T is formed in fp32 (the
+// diagonal blocks' inverses, their products) and R in fp32, but both enter the
+// product U = T R as two bf16 halves, 16 significant bits, without the product
+// of the lower halves. U goes on in bf16 in both kernels. K^T (e^{G_C - G} U)
+// rounds the scaled U; the other kernel rounds the scaled K, which was rounded
+// before, and U. Against 64 bits the output's error is 0.94 to 1.004 times the
+// one-launch kernel's and the state's 0.78 to 1.001 times, over keys from
+// orthogonal to all but parallel (k.k 0.99), beta up to 1 and decay from none
+// to e^-0.5 a token; 8192 tokens of the serving range 0.0038 against 0.0039.
 #include "gdn_device.h"
 #include "../../include/qsa_hip.h"
 

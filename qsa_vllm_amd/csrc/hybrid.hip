@@ -97,7 +97,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // A tile is bound by its VALU work (bf16 conversions, the sigmoid's exp2 and
 // reciprocal at quarter rate: 24 instructions a column and token) and by a
 // chain of load phases, so bf16 roundings are done in pairs and two 8-wave
-// workgroups share a CU at hidden 4096 (110 registers; 16 waves of half the
+// workgroups fit a CU at hidden 4096 (110 registers; 16 waves of half the
 // columns needed 120, one workgroup a CU): 8192 rows 78.6 -> 72 us, 4096 rows
 // 38.6 -> 34 us; the residual add and copy alone take 60 us at 8304 rows.
 // ---------------------------------------------------------------------------
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
 // against 15 us, 1000 rows about equal.
 constexpr int kTokenNormRows = 1024;
 constexpr int kNormRound = 256 * kNormTokens;  // rows of one tile on every CU
-constexpr int kNormTail = 256;
+constexpr int kNormTail = 256;                 // rows past it as single tokens
 constexpr int kTokenNormMaxWaves = 8;  // hidden up to 4096
 
 // Sum over the wave of v[j] for each j < 16: returns the total of rank
@@ -1067,8 +1067,16 @@ extern "C" int qsa_gated_norm(const void* x, int64_t x_stride, const void* resid
     return check_launch("qsa_gated_norm (one workgroup per token)");
   };
   if (rows < kTokenNormRows) return launch_tokens(0);
-  // A few rows past whole rounds of tiles run one workgroup per token too: a
-  // round of 4096-column tiles takes ~25 us however few its tiles are.
+  // Tiles are bound by their CU's VALU work, so the first tile that shares a CU
+  // with another lengthens the launch by 9 to 26 us. At hidden 4096 up to 256
+  // rows past a tile on every CU run one workgroup per token instead, in a
+  // launch before the tiles'. us, all tiles / with it, residual added: 4112 rows
+  // 48.3 / 42.6, 4352 49.1 / 43.4, 8208 97.7 / 79.6, 8448 97.9 / 80.8, 12544
+  // 138.7 / 123.8, 16640 172.6 / 154.6; without: 4112 33.9 / 34.0, 4352 34.7 /
+  // 33.8, 8448 57.9 / 47.9, 12544 73.6 / 70.3, 16640 98.0 / 86.9. It does not pay
+  // in every form past that (512 rows past: 4608 53.1 / 50.3, without residual
+  // 35.0 / 39.3) nor at other sizes: hidden 2048 4112 rows 24.7 / 25.5, 8448 40.0 /
+  // 39.2, without residual 18.1 / 20.5, 27.4 / 28.8; hidden 1024 4112 14.1 / 18.5.
   const int whole = rows / kNormRound * kNormRound;
   if (hidden == 4096 && rows > whole && rows - whole <= kNormTail) {
     a.rows = whole;

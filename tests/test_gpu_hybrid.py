@@ -293,7 +293,7 @@ def test_gated_norm_kernel_against_oracle(rows, hidden, residual):
 def test_gated_norm_row_splits(rows, hidden, residual):
     """The edges of the row split: one workgroup per token below 1024 rows,
     16-token tiles with a partial last tile, and at hidden 4096 up to 256 rows
-    past whole rounds of 4096 rows as single tokens beside the tiles. Every row
+    past whole rounds of 4096 rows as single tokens in a launch of their own. Every row
     is written, none twice: bf16(x + r) is exact."""
     test_gated_norm_kernel_against_oracle(rows, hidden, residual)
 
