@@ -139,3 +139,23 @@ def test_decode_step_bytes_adds_the_three_launches():
     counts = shape.token_topk + wl.seq_lens % shape.compress_ratio
     assert decode_step_bytes(wl, counts) == (indexer_bytes(wl) + want_topk
                                              + attention_bytes(wl, counts))
+
+
+def test_operand_checks_refuse_and_name_the_fault():
+    import torch
+
+    from qsa_vllm_amd.ops import _torch_ops as ops
+
+    t = torch.zeros(6, dtype=torch.int32)
+    assert ops._on_gpu() is None and ops._on_gpu(None, None) is None
+    ops._dtype(t, torch.int32, "x")
+    ops._vector(t, torch.int32, "x", 6)
+    ops._vector(t[:1].expand(1), torch.int32, "x")
+    ops._vector(t[::6], torch.int32, "x")  # one entry: any stride
+    for call, said in ((lambda: ops._on_gpu(None, t), "expected a GPU tensor, got device cpu"),
+                       (lambda: ops._dtype(t, torch.int64, "x"), "x must be torch.int64, got torch.int32"),
+                       (lambda: ops._vector(t.view(2, 3), torch.int32, "x"), "x must be 1-D"),
+                       (lambda: ops._vector(t[::2], torch.int32, "x"), "x must be contiguous"),
+                       (lambda: ops._vector(t, torch.int32, "x", 7), "x has 6 entries, need 7")):
+        with pytest.raises(RuntimeError, match=said):
+            call()
