@@ -46,33 +46,36 @@ inline bool gdn_two_launches(int tokens, int num_seqs, int value_heads, int max_
     const int64_t halves = (pairs + 127) / 128;
     return halves != 2 && halves != 4;
   };
-  const int64_t others = n > 1 ? (tokens - longest) / (n - 1) : 0;  // their mean length
-  if (n > 1 && others < 32) {
-    // Decode sequences among them: the tokens past one per sequence are taken
-    // to be in sequences as long as the longest.
-    const int64_t extra = std::max<int64_t>(tokens - n, 1);
-    const int64_t longs = std::min(n, (extra + longest - 2) / (longest - 1));
-    const int64_t short_pairs = (n - longs) * value_heads;
+  const int64_t others = n > 1 ? (tokens - longest) / (n - 1) : longest;  // their mean length
+  // The tokens past one per sequence, in sequences as long as the longest.
+  const int64_t longs = std::min(n, std::max<int64_t>(tokens - n + longest - 2, 1) / (longest - 1));
+  const int64_t pairs = n * value_heads, long_pairs = longs * value_heads;
+  if (others < 32) {  // decode sequences, most likely, beside the long ones
+    const int64_t short_pairs = pairs - long_pairs;
     if (short_pairs >= 5600 * chunks - 7700) return false;
-    return chunks > 2 || short_pairs >= 512 || rounds_pay(longs * value_heads);
+    return chunks > 2 || short_pairs >= 512 || rounds_pay(long_pairs);
   }
-  if (chunks > 2) return true;
-  const int64_t pairs = n * value_heads;
-  return pairs <= 128 || (others > kGdnChunk && rounds_pay(pairs));
+  if (chunks > 2 || pairs <= 128) return true;
+  if (others <= kGdnChunk) return long_pairs <= 128;  // single chunks, most likely
+  return rounds_pay(pairs) || (long_pairs > 256 && rounds_pay(long_pairs));
 }
 
 // Workspace slots of the two-launch form, one per chunk: sequence `seq`'s chunks
-// take consecutive ones from gdn_first_slot on. Between two sequences of
-// kGdnChunkMin tokens or more seq and start / 16 both grow, so their minimum
-// does; with floor(start / 64) + ceil(len / 64) - 1 <= floor((start + len) / 64),
-// no two chunks share a slot and all are below gdn_slots. A slot per sequence
-// beside those per 64 tokens would serve too, but 900 decode requests beside a
-// prompt of 2000 tokens need 226 this way and 946 that way.
-constexpr int gdn_first_slot(int start, int seq) {
-  return start / kGdnChunk + (seq < start / kGdnChunkMin ? seq : start / kGdnChunkMin);
+// take consecutive ones from gdn_first_slot on. With floor(start / 64) + ceil(len
+// / 64) - 1 <= floor((start + len) / 64), adding anything that grows by one from a
+// chunked sequence to the next keeps their slots apart. The sequence's index
+// does; in a batch of mostly decode sequences its minimum with start / 16 does too
+// (a chunked sequence has 16 tokens) and is bounded by tokens / 16: 900 decode
+// requests beside a prompt of 2000 tokens need 226 slots instead of 946. Unused
+// slots cost next to nothing while there are few, and their workgroups, which
+// end at once, leave room for the others': 7 and one of 1090, 32 value heads, 49 us
+// with them, 52 without.
+constexpr bool gdn_mostly_short(int tokens, int num_seqs) { return num_seqs > tokens / 4; }
+constexpr int gdn_first_slot(int start, int seq, bool mostly_short) {
+  return start / kGdnChunk + (mostly_short && start / kGdnChunkMin < seq ? start / kGdnChunkMin : seq);
 }
 constexpr int64_t gdn_slots(int tokens, int num_seqs) {
-  return (int64_t)tokens / kGdnChunk + (num_seqs < tokens / kGdnChunkMin ? num_seqs : tokens / kGdnChunkMin);
+  return (int64_t)tokens / kGdnChunk + (gdn_mostly_short(tokens, num_seqs) ? tokens / kGdnChunkMin : num_seqs);
 }
 
 // Value columns per workgroup of the walk: the narrowest slices whose workgroups

@@ -109,11 +109,12 @@ __device__ __forceinline__ void chunk_operands(const GdnRecurArgs& a, uint16_t* 
   const int m = lane & 15, g = lane >> 4;
   // The sequence whose chunks cover this slot (none: padding between sequences).
   int seq = -1, start = 0, len = 0;
+  const bool mostly_short = gdn_mostly_short(a.tokens, a.num_seqs);
   for (int i0 = 0; i0 < a.num_seqs && seq < 0; i0 += 64) {
     const int i = min(i0 + lane, a.num_seqs - 1);
     int s0, n;
     const bool chunked = chunked_sequence(a, i, &s0, &n);
-    const int at = slot - gdn_first_slot(s0, i);
+    const int at = slot - gdn_first_slot(s0, i, mostly_short);
     const uint64_t hit = __ballot(chunked && at >= 0 && at < (n + kC - 1) / kC);
     if (hit) {
       const int src = __builtin_ctzll(hit);
@@ -123,7 +124,7 @@ __device__ __forceinline__ void chunk_operands(const GdnRecurArgs& a, uint16_t* 
     }
   }
   if (seq < 0) return;
-  const int c0 = (slot - gdn_first_slot(start, seq)) * kC;
+  const int c0 = (slot - gdn_first_slot(start, seq, mostly_short)) * kC;
   const int nc = min(kC, len - c0);
   const int r = a.value_heads / a.key_heads;
 
@@ -419,7 +420,7 @@ __global__ __launch_bounds__(64 * (SW + 2)) __attribute__((amdgpu_waves_per_eu(2
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g = lane >> 4;
   const int chunks = (len + kC - 1) / kC;
-  const int64_t slot0 = gdn_first_slot(start, seq);
+  const int64_t slot0 = gdn_first_slot(start, seq, gdn_mostly_short(a.tokens, a.num_seqs));
   const int hk = h / (a.value_heads / a.key_heads);
   const int64_t key_stride = (int64_t)a.key_heads * kKeyElems;
   const int64_t val_stride = (int64_t)a.value_heads * kValElems;

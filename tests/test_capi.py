@@ -129,6 +129,7 @@ def test_gdn_recurrence_form_rule():
     # Single-chunk sequences with one of two chunks; few of them are no loss.
     assert not two([64] * 60 + [66]) and not two([40] * 100 + [65]) and not two([16] * 400 + [80])
     assert not two([33] * 24 + [66]) and two([33] * 7 + [128]) and two([40, 128])
+    assert two([1, 40, 60, 70, 85], heads=(16, 32)) and two([64, 100] * 14 + [128]) and not two([64, 96] * 7 + [96, 128])
     # Decode sequences beside prompts.
     for nd, m in ((8, 66), (120, 100), (120, 65), (200, 65), (500, 200), (500, 500), (900, 2000)):
         assert two([1] * nd + [m]), (nd, m)
@@ -163,13 +164,13 @@ def test_gdn_recurrence_workspace_errors_need_no_launch():
 
 
 def test_gdn_recurrence_workspace_counts_chunkable_sequences():
-    """Sequences below 16 tokens take no workspace slot: at most tokens / 16 do."""
+    """In a batch of mostly short sequences no more take a workspace slot than can
+    have 16 tokens."""
     f = _lib.load().qsa_gdn_recurrence_workspace_bytes
     slot = 8 * 32 * 1024 + 16 * 19 * 1024
     assert f(2900, 901, 8, 16, 2000) == (2900 // 64 + 2900 // 16) * slot
     assert f(2112, 113, 8, 16, 2000) == (2112 // 64 + 113) * slot
-    assert f(100, 5, 8, 16, 96) == (1 + 5) * slot
-    assert f(79, 5, 8, 16, 75) == (1 + 4) * slot
+    assert f(400, 100, 8, 16, 301) == (6 + 100) * slot and f(400, 101, 8, 16, 300) == (6 + 25) * slot
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
@@ -196,7 +197,7 @@ int main() {
     for (int i = 0; i < n; ++i) {
       const int len = start[i + 1] - start[i];
       for (int c = 0; len >= qsa::kGdnChunkMin && c * qsa::kGdnChunk < len; ++c) {
-        const int at = qsa::gdn_first_slot(start[i], i) + c;
+        const int at = qsa::gdn_first_slot(start[i], i, qsa::gdn_mostly_short(start[n], n)) + c;
         if (at < 0 || at >= slots || used[at]) { printf("FAIL %d %d\\n", trial, i); return 1; }
         used[at] = 1;
       }
