@@ -27,7 +27,7 @@
 // before, and U. Against 64 bits the output's error is 0.94 to 1.004 times the
 // one-launch kernel's and the state's 0.78 to 1.001 times, over keys from
 // orthogonal to all but parallel (k.k 0.99), beta up to 1 and decay from none
-// to e^-0.5 a token; 8192 tokens of the serving range 0.0038 against 0.0039.
+// to e^-0.5 a token; a prompt of 8192 tokens at the serving decay 0.0038-0.0039 with either.
 #include "gdn_device.h"
 #include "../../include/qsa_hip.h"
 
